@@ -95,16 +95,19 @@ ASX_DEV void cons_from_prim(const Sym3 &g, const Prim &pv, Cons &cv) {
                  pv.entropy, cv);
 }
 
+// The atmosphere at one zone.  Its entropy is evaluated where a zone is set
+// to it (a power on the ideal gas, a temperature solve on a table), not in
+// every zone.
 struct Atmo {
-  double rho, eps, ye, press, temp, entropy, rho_cut;
-  ASX_DEV void set(Prim &pv) const {
+  double rho, eps, ye, press, temp, rho_cut;
+  template <class E>
+  ASX_DEV void set(const E &eos, Prim &pv, Cons &cv, const Sym3 &g) const {
+    double eps = this->eps; // clamped to the EOS's range, as by the reference
+    const double entropy = eos.kappa_near(rho, eps, ye, temp);
     pv.rho = rho; pv.eps = eps; pv.Ye = ye; pv.press = press;
     pv.temperature = temp; pv.entropy = entropy;
     pv.vel[0] = pv.vel[1] = pv.vel[2] = 0.0;
     pv.w_lor = 1.0;
-  }
-  ASX_DEV void set(Prim &pv, Cons &cv, const Sym3 &g) const {
-    set(pv);
     const double sqrt_detg = sqrt(det3(g));
     cv.dens = sqrt_detg * rho;
     cv.mom[0] = cv.mom[1] = cv.mom[2] = 0.0;
@@ -154,8 +157,7 @@ template <class E> ASX_DEV Atmo make_atmo(const E &eos, const C2PArgs &a, double
     eps_atm = smin(smax(eos.eps_min, eps_atm), eos.eps_max);
     press_atm = eos.press_re(rho_atm, eps_atm, a.Ye_atmo);
   }
-  const double entropy_atm = eos.kappa_re(rho_atm, eps_atm, a.Ye_atmo);
-  return Atmo{rho_atm, eps_atm, a.Ye_atmo, press_atm, temp_atm, entropy_atm,
+  return Atmo{rho_atm, eps_atm, a.Ye_atmo, press_atm, temp_atm,
               rho_atm * (1 + a.atmo_tol)};
 }
 
@@ -477,7 +479,7 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
   cv.DEnt = cv.dens * pv.entropy;
   if (pv.rho < atmo.rho_cut) {
     rep.status = ST_SUCCESS; rep.set_atmo = true; rep.adjust_cons = true;
-    atmo.set(pv, cv, glo);
+    atmo.set(eos, pv, cv, glo);
     return;
   }
   prims_floors(eos, atmo, a, pv, cv, glo, rep);
@@ -491,13 +493,13 @@ template <class E> struct PalF {
   const Atmo &atmo;
   const C2PArgs &a;
   double q, r, s, t, dens, ye;
-  // the table's temperature cell of the previous evaluation (successive
-  // Brent iterates of one zone move T little; the solve is exact either way)
-  mutable int thint = -1;
+  // the table's cell of the previous evaluation (successive Brent iterates
+  // of one zone move rho and T little; the solve is exact either way)
+  typename E::Cell &cell;
   ASX_DEV double operator()(double x) const {
     double Wm2 = 1.0 - (x * x * r + (2.0 * x + s) * t * t) / (x * x * (x + s) * (x + s));
     Wm2 = fmin(fmax(Wm2, 1e-10), 1);
-    const double W = pow(Wm2, -0.5);
+    const double W = 1.0 / sqrt(Wm2);
     const double rho = dens / W;
     double eps = W - 1.0 + (1.0 - W * W) * x / W +
                  W * (q - s + t * t / (2 * x * x) + s / (2 * W * W));
@@ -505,7 +507,7 @@ template <class E> struct PalF {
       eps = smax(eps, atmo.eps);
       eps = smin(eps, eos.eps_max);
     }
-    const double P = eos.press_re(rho, eps, ye, &thint);
+    const double P = eos.press_re(rho, eps, ye, cell);
     return (x - (1.0 + eps + P / rho) * W);
   }
 };
@@ -578,11 +580,13 @@ ASX_DEV void brent(const F &fn, double a, double b, double fa0, double fb0, doub
   rb = c;
 }
 
-// Palenzuela 1D, c2p_1DPalenzuela.hxx:306-556
+// Palenzuela 1D, c2p_1DPalenzuela.hxx:306-556.  tseed: the temperature a
+// table's first solve starts its search from (any value; no result depends
+// on it).
 template <class E>
 ASX_DEV void palenzuela_solve(const E &eos, const Atmo &atmo, const C2PArgs &a,
                               Prim &pv, Cons &cv, const Sym3 &glo, Report &rep,
-                              double xguess = -1.0, double xrel = 0.0,
+                              double tseed, double xguess = -1.0, double xrel = 0.0,
                               bool miss_fails = false) {
   rep.iters = 0;
   rep.adjust_cons = false;
@@ -620,7 +624,9 @@ ASX_DEV void palenzuela_solve(const E &eos, const Atmo &atmo, const C2PArgs &a,
   const double s = Bsq / cv.dens;
   const double r = Ssq / pow2(cv.dens);
   const double t = BiSi / pow(cv.dens, 3. / 2.);
-  const PalF<E> fn{eos, atmo, a, q, r, s, t, cv.dens, cv.DYe / cv.dens};
+  typename E::Cell cell;
+  eos.start_cell(cell, cv.DYe / cv.dens, tseed);
+  const PalF<E> fn{eos, atmo, a, q, r, s, t, cv.dens, cv.DYe / cv.dens, cell};
   const double xa = smax(1e-10, 1.0 + q - s);
   double xb = 2.0 + 2.0 * q - s;
   double lo = xa, hi = xb, flo = 0.0, fhi = 0.0;
@@ -661,7 +667,7 @@ ASX_DEV void palenzuela_solve(const E &eos, const Atmo &atmo, const C2PArgs &a,
   {
     double Wm2 = 1.0 - (x * x * r + (2.0 * x + s) * t * t) / (x * x * (x + s) * (x + s));
     Wm2 = fmin(fmax(Wm2, 1e-10), 1);
-    const double W = pow(Wm2, -0.5);
+    const double W = 1.0 / sqrt(Wm2);
     pv.rho = cv.dens / W;
     pv.eps = W - 1.0 + (1.0 - W * W) * x / W +
              W * (q - s + t * t / (2 * x * x) + s / (2.0 * W * W));
@@ -671,7 +677,7 @@ ASX_DEV void palenzuela_solve(const E &eos, const Atmo &atmo, const C2PArgs &a,
     }
     vel_from_Z(x * pv.rho * W, W, Bsq, BiSi, cv, gup, glo, a.use_z, pv);
     pv.Ye = cv.DYe / cv.dens;
-    eos.state_re(pv.rho, pv.eps, pv.Ye, pv.press, pv.temperature, pv.entropy, &fn.thint);
+    eos.state_re(pv.rho, pv.eps, pv.Ye, pv.press, pv.temperature, pv.entropy, cell);
     pv.B[0] = cv.dB[0]; pv.B[1] = cv.dB[1]; pv.B[2] = cv.dB[2];
   }
   if (pv.rho <= 0.0) {
@@ -703,7 +709,7 @@ ASX_DEV void palenzuela_solve(const E &eos, const Atmo &atmo, const C2PArgs &a,
   cv.DEnt = cv.dens * pv.entropy;
   if (pv.rho < atmo.rho_cut) {
     rep.status = ST_SUCCESS; rep.set_atmo = true; rep.adjust_cons = true;
-    atmo.set(pv, cv, glo);
+    atmo.set(eos, pv, cv, glo);
     return;
   }
   prims_floors(eos, atmo, a, pv, cv, glo, rep);
@@ -813,7 +819,7 @@ ASX_DEV void entropy_solve(const E &eos, const Atmo &atmo, const C2PArgs &a, Pri
            cv.dens;
   if (pv.rho < atmo.rho_cut) {
     rep.status = ST_SUCCESS; rep.set_atmo = true; rep.adjust_cons = true;
-    atmo.set(pv, cv, glo);
+    atmo.set(eos, pv, cv, glo);
     return;
   }
   prims_floors(eos, atmo, a, pv, cv, glo, rep);
@@ -884,12 +890,9 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
     seed.rho = in.saved_rho;
     seed.eps = in.saved_eps;
     seed.Ye = in.saved_Ye;
-    {
-      // p and the entropy of the saved state; the EOS takes eps by reference
-      // (a table may clamp it), the seed keeps the value as loaded
-      double e = in.saved_eps, temp;
-      eos.state_re(in.saved_rho, e, in.saved_Ye, seed.press, temp, seed.entropy);
-    }
+    // the seed's pressure and entropy are read nowhere: Noble takes its own
+    // pressure, the BH-interior and atmosphere paths set both
+    seed.press = seed.entropy = __builtin_nan("");
     seed.temperature = in.temperature;
     seed.vel[0] = v_up[0]; seed.vel[1] = v_up[1]; seed.vel[2] = v_up[2];
     seed.w_lor = sqrt(1.0 + zsq);
@@ -900,8 +903,7 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
   bool call_c2p = true;
   if (cv.dens <= sqrt_detg * atmo.rho_cut) {
     pv.B[0] = Bup[0]; pv.B[1] = Bup[1]; pv.B[2] = Bup[2];
-    atmo.set(pv, cv, glo);
-    atmo.set(seed);
+    atmo.set(eos, pv, cv, glo);
     code = ASX_C2P_FLAG_ATMO;
     call_c2p = false;
   }
@@ -924,10 +926,10 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
       if (prime == ASX_C2P_NOBLE)
         noble_solve<SEEDLESS>(eos, atmo, a, pv, seed, cv, glo, rep1, zguess, vguess);
       else if (prime == ASX_C2P_ENTROPY) entropy_solve(eos, atmo, a, pv, cv, glo, rep1);
-      else palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, zguess, vguess, PRIME >= 0);
+      else palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, in.temperature, zguess, vguess, PRIME >= 0);
     } else {
       (void)prime; // Noble needs the ideal-fluid Gamma; refused for tables at the C ABI
-      palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, zguess, vguess, PRIME >= 0);
+      palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, in.temperature, zguess, vguess, PRIME >= 0);
     }
     out.iters = rep1.iters;
     if (PRIME >= 0 && rep1.failed()) return false;
@@ -935,10 +937,10 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
       code = ASX_C2P_FLAG_SECOND;
       if constexpr (std::is_same<E, IdealGas>::value) {
         if (a.second == ASX_C2P_NOBLE) noble_solve(eos, atmo, a, pv, seed, cv, glo, rep2);
-        else if (a.second == ASX_C2P_PALENZUELA) palenzuela_solve(eos, atmo, a, pv, cv, glo, rep2);
+        else if (a.second == ASX_C2P_PALENZUELA) palenzuela_solve(eos, atmo, a, pv, cv, glo, rep2, in.temperature);
         else if (a.second == ASX_C2P_ENTROPY) entropy_solve(eos, atmo, a, pv, cv, glo, rep2);
       } else {
-        if (a.second == ASX_C2P_PALENZUELA) palenzuela_solve(eos, atmo, a, pv, cv, glo, rep2);
+        if (a.second == ASX_C2P_PALENZUELA) palenzuela_solve(eos, atmo, a, pv, cv, glo, rep2, in.temperature);
       }
     }
     bool failed = rep1.failed() && rep2.failed();
@@ -959,7 +961,7 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
       } else {
         for (int i = 0; i < 3; ++i) cv.dB[i] = sqrt_detg * Bup[i];
         pv.B[0] = Bup[0]; pv.B[1] = Bup[1]; pv.B[2] = Bup[2];
-        atmo.set(pv, cv, glo);
+        atmo.set(eos, pv, cv, glo);
       }
     }
     if ((mask_local != 1.0) && flag_local) bh_interior<true>(eos, atmo, a, pv, cv, glo);

@@ -90,45 +90,162 @@ struct TabEOS {
   ASX_DEV double xmin1() const { return ax[1][0]; }
   ASX_DEV double xmax1() const { return ax[1][n[1] - 1]; }
 
-  // logtemp_from_valid_rho_eps_ye (eos_3p_tabulated3d.hxx:186-218).  hint
-  // (optional) is the T cell of the previous solve for the same zone: when
-  // that cell, away from the table's ends, still brackets the value, the
-  // root is solved there with two node values instead of the end values and
-  // the bisection.  For a table whose eps grows with T the bracketing cell is
-  // unique, so the result is the same bits either way.
-  ASX_DEV double logtemp_re(double rho, double &eps, double ye, int *hint = nullptr) const {
+  // logtemp_from_valid_rho_eps_ye (eos_3p_tabulated3d.hxx:186-218)
+  ASX_DEV double logtemp_re(double rho, double &eps, double ye) const {
     const double r = crho(rho);
     eps = fmax(eps + shift, eps_min + shift) - shift;
     const double lrho = log(r);
     const double leps = log(eps + shift);
-    if (hint && *hint >= 0 && *hint <= n[1] - 3) {
-      const int i0 = find(0, lrho), i2 = find(2, ye), h = *hint;
-      const int s1 = NV * n[0], s2 = NV * n[0] * n[1];
-      const double *p = tab + EPS + NV * i0 + s2 * i2;
-      const double r0 = ax[0][i0], r1 = ax[0][i0 + 1];
-      const double y0 = ax[2][i2], y1 = ax[2][i2 + 1];
-      const double eh = enode(p + s1 * h, s2, r0, r1, y0, y1, lrho, ye);
-      const double eh1 = enode(p + s1 * (h + 1), s2, r0, r1, y0, y1, lrho, ye);
-      // at h = 0 the bisection takes the end value, equal to E_0: strictly
-      // above it, no clamp applies
-      if (eh <= leps && leps < eh1 && (h > 0 || leps > eh)) {
-        const double t0 = ax[1][h], t1 = ax[1][h + 1];
-        return t0 + (leps - eh) * (t1 - t0) / (eh1 - eh);
-      }
-    }
     const double vmin = interp(EPS, lrho, xmin1(), ye);
     const double vmax = interp(EPS, lrho, xmax1(), ye);
     if (leps <= vmin) {
       eps = exp(vmin) - shift;
-      if (hint) *hint = -1;
       return xmin1();
     }
     if (leps >= vmax) {
       eps = exp(vmax) - shift;
-      if (hint) *hint = -1;
       return xmax1();
     }
-    return logtemp_nodes(lrho, leps, ye, vmin, vmax, hint);
+    return logtemp_nodes(lrho, leps, ye, vmin, vmax);
+  }
+  // The table cell of a zone's previous solve, kept in registers between the
+  // solves of one zone: node indices (i1 < 0: none yet), the cell's position
+  // and inverse width on each axis, and per corner [Ye][T][rho]
+  // log(eps + shift) and log p.
+  struct Cell {
+    int i0 = -1, i1 = -1, i2 = 0;
+    double r0, ri, t0, dt, ly; // log rho: low node, 1 / width; log T: low node, width; Ye weight
+    double e[2][2][2], p[2][2][2];
+  };
+  // Start of a zone's solves: its Ye, and a temperature near which to look.
+  ASX_DEV void start_cell(Cell &c, double ye, double temp) const {
+    c.i2 = find(2, ye);
+    c.ly = (ye - ax[2][c.i2]) / (ax[2][c.i2 + 1] - ax[2][c.i2]);
+    c.i1 = find(1, log(ctemp(temp)));
+    c.i0 = -1;
+  }
+  ASX_DEV void load_cell(Cell &c, int i0, int i1) const {
+    const int s1 = NV * n[0], s2 = NV * n[0] * n[1];
+    const double *q = tab + NV * i0 + s1 * i1 + s2 * c.i2;
+    if (c.i0 != i0) {
+      c.r0 = ax[0][i0];
+      c.ri = 1.0 / (ax[0][i0 + 1] - c.r0);
+    }
+    c.t0 = ax[1][i1];
+    c.dt = ax[1][i1 + 1] - c.t0;
+    c.i0 = i0;
+    c.i1 = i1;
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const double *v = q + y * s2 + t * s1 + r * NV; // log p and log eps are adjacent
+          c.p[y][t][r] = v[PRESS];
+          c.e[y][t][r] = v[EPS];
+        }
+  }
+  // p and log T from (rho, eps, Ye) with the zone's previous cell as the
+  // starting point: the same root as logtemp_re's for a table whose eps
+  // grows with T along each (rho, Ye) line (the bracketing cell is then
+  // unique), to rounding.  A zone's consecutive solves (the Brent iterates,
+  // then the final state) move rho and eps by less and less, so the cell
+  // they end in repeats: its corner values stay in registers and a solve
+  // inside it reads no memory.  When the root has left it, the next cell is
+  // predicted from the cell's slope d eps / d T (exact for a thermal energy
+  // linear in T, so it usually lands on the cell or beside it) and checked
+  // at its own nodes; a miss is searched outwards from there by doubling
+  // steps, then bisected.
+  // Bound by the latency of dependent table reads: some lane of a wavefront
+  // leaves its cell in almost every iteration, and a search from scratch
+  // costs the whole wavefront eight dependent probes.  Con2prim of 1 000 003
+  // zones on the 234 x 180 x 50 table: 2.75 ms with the search from scratch
+  // outside the previous T cell, 0.79 ms with this (table reads per
+  // wavefront 1490 -> 436, waves waiting 74 % -> 34 % of their time);
+  // keeping the corners alone, without the prediction, left it at 2.70.
+  ASX_DEV void solve_re(double rho, double &eps, Cell &c, double &lrho, double &lt,
+                        double &press) const {
+    const double r = crho(rho);
+    eps = fmax(eps + shift, eps_min + shift) - shift;
+    lrho = log(r);
+    const double es = eps + shift, leps = log(es);
+    const int i0 = find(0, lrho), last = n[1] - 1;
+    if (c.i0 != i0) load_cell(c, i0, c.i1);
+    const double lr = (lrho - c.r0) * c.ri;
+    auto mix = [&](const double (&v)[2][2][2], int t) {
+      const double a0 = (v[0][t][1] - v[0][t][0]) * lr + v[0][t][0];
+      const double a1 = (v[1][t][1] - v[1][t][0]) * lr + v[1][t][0];
+      return (a1 - a0) * c.ly + a0;
+    };
+    double elo = mix(c.e, 0), ehi = mix(c.e, 1);
+    // outside [elo, ehi): every lane of the wavefront that has left its cell
+    auto below = [&] { return !(elo <= leps); };
+    auto above = [&] { return !(leps < ehi); };
+    if ((below() && c.i1 > 0) || (above() && c.i1 < last - 1)) {
+      // eps linear in T through the cell's nodes, in single precision
+      const float k = 1.44269504f;
+      const float dlo = __builtin_amdgcn_exp2f(k * (float)(elo - leps));
+      const float dhi = __builtin_amdgcn_exp2f(k * (float)(ehi - leps));
+      const float th = __builtin_amdgcn_exp2f(k * (float)c.dt);
+      // T / T_lo at the target
+      const float x = 1.0f + (1.0f - dlo) * (th - 1.0f) / (dhi - dlo);
+      const float step = __builtin_amdgcn_logf(fmaxf(x, 1e-30f)) / (k * (float)c.dt);
+      int j = c.i1 + (int)fminf(fmaxf(floorf(step), -(float)last), (float)last);
+      j = below() ? min(j, c.i1 - 1) : max(j, c.i1 + 1); // past the cell it left
+      j = min(max(j, 0), last - 1);
+      load_cell(c, i0, j);
+      elo = mix(c.e, 0);
+      ehi = mix(c.e, 1);
+      if ((below() && j > 0) || (above() && j < last - 1)) {
+        const int s1 = NV * n[0];
+        const double *row = tab + EPS + NV * i0 + s1 * n[1] * c.i2;
+        auto node = [&](int m) {
+          const double *q = row + s1 * m;
+          const int s2 = s1 * n[1];
+          const double a0 = (q[NV] - q[0]) * lr + q[0];
+          const double a1 = (q[s2 + NV] - q[s2]) * lr + q[s2];
+          return (a1 - a0) * c.ly + a0;
+        };
+        int lo = j, hi = j + 1, d = 1;
+        if (below()) {
+          while (lo > 0 && below()) {
+            hi = lo;
+            lo = max(lo - d, 0);
+            d *= 2;
+            elo = node(lo);
+          }
+        } else {
+          while (hi < last && above()) {
+            lo = hi;
+            hi = min(hi + d, last);
+            d *= 2;
+            ehi = node(hi);
+          }
+        }
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (node(mid) <= leps) lo = mid;
+          else hi = mid;
+        }
+        load_cell(c, i0, lo);
+        elo = mix(c.e, 0);
+        ehi = mix(c.e, 1);
+      }
+    }
+    double f; // log T weight in the cell
+    if (c.i1 == 0 && leps <= elo) { // at or below the table's lowest T
+      eps = exp(elo) - shift;
+      f = 0.0;
+    } else if (c.i1 == last - 1 && leps >= ehi) {
+      eps = exp(ehi) - shift;
+      f = 1.0;
+    } else {
+      f = (leps - elo) / (ehi - elo);
+    }
+    lt = c.t0 + f * c.dt;
+    const double b0 = mix(c.p, 0), b1 = mix(c.p, 1);
+    press = exp((b1 - b0) * f + b0);
   }
   // E_j at the node row q of the T axis: log(eps + shift) interpolated in
   // log rho, then in Ye (the reference's order)
@@ -149,7 +266,7 @@ struct TabEOS {
   // iteration on the same function stops within 2 eps |lt| + 1e-14 of this
   // root, after about twice as many dependent steps of twice the reads.
   ASX_DEV double logtemp_nodes(double lrho, double leps, double ye, double vmin,
-                               double vmax, int *hint = nullptr) const {
+                               double vmax) const {
     const int i0 = find(0, lrho), i2 = find(2, ye);
     const int s1 = NV * n[0], s2 = NV * n[0] * n[1];
     const double *p = tab + EPS + NV * i0 + s2 * i2;
@@ -168,7 +285,6 @@ struct TabEOS {
         ehi = em;
       }
     }
-    if (hint) *hint = lo;
     const double t0 = ax[1][lo], t1 = ax[1][hi];
     return t0 + (leps - elo) * (t1 - t0) / (ehi - elo);
   }
@@ -176,10 +292,15 @@ struct TabEOS {
   ASX_DEV double press_rt(double rho, double temp, double ye) const {
     return exp(interp(PRESS, log(rho), log(temp), ye));
   }
-  ASX_DEV double press_re(double rho, double &eps, double ye, int *hint = nullptr) const {
+  ASX_DEV double press_re(double rho, double &eps, double ye) const {
     const double lr = log(crho(rho));
-    const double lt = logtemp_re(rho, eps, ye, hint);
+    const double lt = logtemp_re(rho, eps, ye);
     return exp(interp(PRESS, lr, lt, ye));
+  }
+  ASX_DEV double press_re(double rho, double &eps, double, Cell &c) const {
+    double lr, lt, press;
+    solve_re(rho, eps, c, lr, lt, press);
+    return press;
   }
   ASX_DEV double eps_rt(double rho, double temp, double ye) const {
     return exp(interp(EPS, log(crho(rho)), log(ctemp(temp)), ye)) - shift;
@@ -201,9 +322,9 @@ struct TabEOS {
   // where that clamp applied, the later solves may land an ulp away from
   // the table edge, which is the only difference
   ASX_DEV void state_re(double rho, double &eps, double ye, double &press, double &temp,
-                        double &kap, int *hint = nullptr) const {
-    const double lt = logtemp_re(rho, eps, ye, hint);
-    press = exp(interp(PRESS, log(crho(rho)), lt, ye));
+                        double &kap, Cell &c) const {
+    double lr, lt;
+    solve_re(rho, eps, c, lr, lt, press);
     temp = exp(lt);
     kap = entropy_rt(rho, temp, ye);
   }
@@ -214,6 +335,14 @@ struct TabEOS {
   // kappa_from_valid_rho_eps_ye (:331-336): the entropy at T(rho, eps, Ye)
   ASX_DEV double kappa_re(double rho, double &eps, double ye) const {
     return entropy_rt(rho, temp_re(rho, eps, ye), ye);
+  }
+  // the same where the temperature is known to lie near `temp`
+  ASX_DEV double kappa_near(double rho, double &eps, double ye, double temp) const {
+    Cell c;
+    start_cell(c, ye, temp);
+    double press, t, kap;
+    state_re(rho, eps, ye, press, t, kap, c);
+    return kap;
   }
   // eps_from_valid_rho_press_ye is refused by the reference for tables;
   // the callers that reach it (pressure atmosphere, use_temperature = no)

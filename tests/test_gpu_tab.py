@@ -212,6 +212,49 @@ def test_c2p_batch_ye_table_matches_oracle():
     _c2p_case(dtab, htab, 4000, 21)
 
 
+@pytest.mark.parametrize("shape", [(2, 2, 2), (3, 3, 2), (5, 4, 3), (40, 9, 4)])
+@pytest.mark.parametrize("tseed", [0.0, 1e300, float("nan")])
+def test_c2p_batch_ye_small_tables_any_seed_temperature(shape, tseed):
+    """The temperature search between a zone's solves (start cell from the
+    seed temperature, prediction, outward search, the ends of the T axis) on
+    the smallest tables, from any starting temperature, against the oracle.
+    Both stop within dx = 2^-33 x of the root, so they differ by at most
+    2 dx; W(x) moves by W^3 v^2 dx / x, which bounds rho = D / W, and eps(x)
+    by (W + 2 W^3) dx (its x and W terms), each taken twice over."""
+    torch = _torch()
+    tab = tabeos.build(*shape)
+    dtab, htab = tabeos.Table(tab, device="cuda"), tabeos.Table(tab, device=None)
+    par_d, par_h = _par(dtab), _par(htab)
+    nz = 777
+    prim, g = zones.make_batch_ye(nz, 31, (1e-12, 1e-4), (0.05, 80.0), (0.06, 0.5))
+    L, O = _L(), oracle.lib()
+    cons, thermo = np.zeros((9, nz)), np.zeros((2, nz))
+    abi.check("orc_prim2con_batch_ye", O.orc_prim2con_batch_ye(
+        nz, prim.ctypes.data, g.ctypes.data, cons.ctypes.data, thermo.ctypes.data,
+        C.byref(par_h)))
+    seed = np.ascontiguousarray(np.stack([prim[0], thermo[0], prim[3], prim[4], prim[5], prim[2],
+                                          np.full(nz, tseed)]))
+    out, flag, iters = np.zeros((9, nz)), np.zeros(nz), np.zeros(nz, dtype=np.int32)
+    abi.check("orc_c2p_batch_ye", O.orc_c2p_batch_ye(
+        nz, cons.ctypes.data, g.ctypes.data, seed.ctypes.data, out.ctypes.data,
+        flag.ctypes.data, iters.ctypes.data, C.byref(par_h)))
+    od = torch.empty((9, nz), dtype=torch.float64, device="cuda")
+    fd = torch.empty(nz, dtype=torch.float64, device="cuda")
+    idd = torch.empty(nz, dtype=torch.int32, device="cuda")
+    cd, gd, sd = _dev(cons), _dev(g), _dev(seed)
+    abi.check("asx_c2p_batch_ye", L.asx_c2p_batch_ye(
+        nz, _p(cd), _p(gd), _p(sd), _p(od), _p(fd), _p(idd), C.byref(par_d), None))
+    torch.cuda.synchronize()
+    got = od.cpu().numpy()
+    assert np.array_equal(fd.cpu().numpy(), flag)
+    ok = flag == 1
+    assert ok.mean() > 0.9
+    rho, eps, press, w = (out[r, ok] for r in (0, 1, 2, 6))
+    x = (1 + eps + press / rho) * w
+    assert (np.abs(got[0, ok] - rho) <= 2.0 ** -31 * w ** 2 * rho).all()
+    assert (np.abs(got[1, ok] - eps) <= 2.0 ** -31 * (w + 2 * w ** 3) * x).all()
+
+
 def test_c2p_batch_ye_ideal_gas_matches_oracle():
     dtab, htab = _tables()
     _c2p_case(dtab, htab, 4000, 22, ideal=True)
