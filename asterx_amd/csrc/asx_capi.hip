@@ -1150,7 +1150,11 @@ asx_status asx_bc_fill(const asx_patch *pt, int32_t slot, int32_t kind, void *st
     if (kind == ASX_BC_LINEAR && pt->n[d] + c < 2) return ASX_ERR_SIZE;
     if (kind == ASX_BC_PERIODIC && pt->n[d] < pt->ng) return ASX_ERR_SIZE;
   }
-  return dev_status(timed(ASX_KC_BC, (hipStream_t)stream, [&] { return launch_bc(kpatch(pt), slot, kind, (hipStream_t)stream); }));
+  BCList L;
+  L.nf = 1;
+  L.g[0] = pt->gf[slot].data;
+  L.cent[0] = centering(slot);
+  return dev_status(timed(ASX_KC_BC, (hipStream_t)stream, [&] { return launch_bc_many(kpatch(pt), L, kind, (hipStream_t)stream); }));
 }
 
 asx_status asx_timing_enable(int32_t on) {
@@ -2019,10 +2023,10 @@ enum BatchKind {
   BK_FACE = 0,   // + d: faces, tiles of the face variant
   BK_AUX = 3,    // vertices, two layers into the ghosts
   BK_UPDATE = 4, // interior vertices, tiles of the update variant
-  BK_BC = 5,     // + d: ghost layers normal to d
-  BK_UBSTAG = 8, // + d: interior faces of the caller's dB_stag
-  BK_C2P = 11,   // interior cells
-  BK_COUNT = 12
+  BK_BC = 5,     // ghost layers (bc_point's workgroups)
+  BK_UBSTAG = 6, // + d: interior faces of the caller's dB_stag
+  BK_C2P = 9,    // interior cells
+  BK_COUNT = 10
 };
 
 struct BatchLaunch {
@@ -2124,13 +2128,10 @@ asx_status plan_launch(asx_batch *b, int k, int v, BatchLaunch **out) {
         bb.cnt[q] = bx.cnt[q];
       }
       update_tile_extent(v, tile);
-    } else if (k >= BK_BC && k < BK_BC + 3) {
-      const int d = k - BK_BC; // bc_point's pass normal to d, widest centering
-      for (int q = 0; q < 3; ++q) {
-        bb.lo[q] = 0;
-        bb.cnt[q] = q > d ? pt.n[q] + 1 : pt.n[q] + 2 * pt.ng + 1;
-      }
-      bb.cnt[d] = 2 * pt.ng;
+    } else if (k == BK_BC) { // whole workgroups; bc_point knows their points
+      bb.lo[0] = bb.lo[1] = bb.lo[2] = 0;
+      bb.cnt[0] = 256 * bc_blocks(pt.n, pt.ng);
+      bb.cnt[1] = bb.cnt[2] = 1;
     } else if (k >= BK_UBSTAG && k < BK_UBSTAG + 3) {
       const int d = k - BK_UBSTAG;
       const int halo[3] = {0, 0, 0};
@@ -2221,16 +2222,12 @@ asx_status plan_bc(asx_batch *b, const KPatch *T, const int *slots, int n, hipSt
     S.slot[q] = slots[q];
     S.cent[q] = centering(slots[q]);
   }
-  for (int d = 0; d < 3; ++d) {
-    BatchLaunch *L;
-    asx_status st;
-    if ((st = plan_launch(b, BK_BC + d, 0, &L))) return st;
-    if ((st = dev_status(timed(ASX_KC_BC, str, [&] {
-           return launch_bc_batch(d, T, S, L->map, L->nmap, b->bc_kind, str);
-         }))))
-      return st;
-  }
-  return ASX_OK;
+  BatchLaunch *L;
+  asx_status st;
+  if ((st = plan_launch(b, BK_BC, 0, &L))) return st;
+  return dev_status(timed(ASX_KC_BC, str, [&] {
+    return launch_bc_batch(T, S, L->map, L->nmap, b->bc_kind, str);
+  }));
 }
 
 asx_status plan_stage(asx_batch *b, int s, hipStream_t str) {
@@ -2336,8 +2333,8 @@ asx_status plan_persist_prepare(asx_batch *b) {
   PersistArgs a;
   std::memset(&a, 0, sizeof(a));
   for (int d = 0; d < 3; ++d)
-    if (!list(BK_FACE + d, 0, a.face[d]) || !list(BK_BC + d, 0, a.bc[d])) return st;
-  if (!list(BK_AUX, 0, a.aux) || !list(BK_UPDATE, 1, a.update) || !list(BK_C2P, 0, a.c2p))
+    if (!list(BK_FACE + d, 0, a.face[d])) return st;
+  if (!list(BK_BC, 0, a.bc) || !list(BK_AUX, 0, a.aux) || !list(BK_UPDATE, 1, a.update) || !list(BK_C2P, 0, a.c2p))
     return st;
   a.A = plan_flux_args(&par);
   a.R = R;

@@ -13,10 +13,14 @@ namespace asx {
 struct Box {
   int lo[3], cnt[3];
   ASX_DEV int64_t total() const { return (int64_t)cnt[0] * cnt[1] * cnt[2]; }
+  // point t < total(), which is below 2^31 (a patch's points are): 32-bit
+  // divisions, a fifth of the instructions of the 64-bit ones
   ASX_DEV void ijk(int64_t t, int &i, int &j, int &k) const {
-    i = lo[0] + (int)(t % cnt[0]);
-    j = lo[1] + (int)((t / cnt[0]) % cnt[1]);
-    k = lo[2] + (int)(t / ((int64_t)cnt[0] * cnt[1]));
+    const unsigned u = (unsigned)t, nx = (unsigned)cnt[0], ny = (unsigned)cnt[1];
+    const unsigned r = u / nx, z = r / ny;
+    i = lo[0] + (int)(u - r * nx);
+    j = lo[1] + (int)(r - z * ny);
+    k = lo[2] + (int)z;
   }
   __host__ int64_t htotal() const { return (int64_t)cnt[0] * cnt[1] * cnt[2]; }
   __host__ dim3 grid() const { return dim3((unsigned)((htotal() + 255) / 256)); }
@@ -280,7 +284,6 @@ hipError_t launch_sources(const KPatch &P, const Box &B, const RhsArgs &A,
 hipError_t launch_rhs(const KPatch &P, const RhsArgs &A, hipStream_t s);
 hipError_t launch_lincomb(double *dst, int64_t np, double scale, int nsrc,
                           const double *fac, double *const *src, hipStream_t s);
-hipError_t launch_bc(const KPatch &P, int slot, int kind, hipStream_t s);
 // Grid functions filled by one multi-field boundary launch.
 constexpr int kMaxBC = 64;
 struct BCList {
@@ -288,6 +291,19 @@ struct BCList {
   int cent[kMaxBC];
   int nf;
 };
+// Work-items of the ghost layers normal to axis d, for the widest centering
+// (vertex on every axis): the full extent on the axes before d, the interior
+// after it, so that the three sets are disjoint.  Each set starts a new
+// workgroup of 256: bc_blocks(d) workgroups.
+__host__ __device__ inline int bc_blocks(const int n[3], int ng, int d) {
+  int w[3] = {n[0] + 2 * ng + 1, n[1] + 2 * ng + 1, n[2] + 2 * ng + 1};
+  for (int a = d + 1; a < 3; ++a) w[a] = n[a] + 1;
+  w[d] = 2 * ng;
+  return (w[0] * w[1] * w[2] + 255) / 256;
+}
+__host__ __device__ inline int bc_blocks(const int n[3], int ng) {
+  return bc_blocks(n, ng, 0) + bc_blocks(n, ng, 1) + bc_blocks(n, ng, 2);
+}
 hipError_t launch_bc_many(const KPatch &P, const BCList &L, int kind, hipStream_t s);
 hipError_t launch_update(const KPatch &P, const RhsArgs &A, const StatePtrs &u0,
                          const StatePtrs &out, double c0, double c1, double c2,
@@ -337,8 +353,8 @@ hipError_t launch_update_batch(const KPatch *tab, const StatePtrs *u0, const Sta
                                int variant, hipStream_t s);
 // boundary fill along axis d; map chunks are 256-point blocks of the 2 ng
 // ghost layers normal to d, sized for the widest centering
-hipError_t launch_bc_batch(int d, const KPatch *tab, const BCSlots &L, const BatchRef *map,
-                           int nmap, int kind, hipStream_t s);
+hipError_t launch_bc_batch(const KPatch *tab, const BCSlots &L, const BatchRef *map, int nmap,
+                           int kind, hipStream_t s);
 // con2prim of the patch interiors; zbase[p] = first global zone of patch p
 // (np + 1 entries), the queue holds global zone indices
 hipError_t launch_con2prim_main_batch(const KPatch *tab, const int *zbase, int np,
@@ -367,7 +383,7 @@ struct PersistArgs {
   double c0, c1, c2;
   IdealGas eos;
   C2PArgs ca;
-  BatchList face[3], aux, update, bc[3], c2p;
+  BatchList face[3], aux, update, bc, c2p;
   BCSlots state, prims; // grid functions filled after the update / con2prim
   int bc_kind;
   const int *zbase;

@@ -5,10 +5,10 @@
 //   1. faces normal to x, y, z and the vertex auxiliaries of every patch
 //      (independent of one another; the con2prim queue count is cleared)
 //   2. the fused RHS + RK combination of every patch
-//   3. boundary fill of the 11 evolved fields, axis x, then y, then z
+//   3. boundary fill of the 11 evolved fields
 //   4. con2prim, Noble primary, failures queued by a wavefront ballot
 //   5. the queued zones through the full chain
-//   6. boundary fill of the 12 synced primitives, axis x, then y, then z
+//   6. boundary fill of the 12 synced primitives
 // The work of each phase is the plan's (patch, chunk) list; XCD x (the
 // workgroups with blockIdx.x % 8 == x) takes one contiguous run of it, so
 // neighbouring tiles of a patch share one L2.  The bodies are the device
@@ -73,13 +73,12 @@ template <int ORD> ASX_ITEM void update_item(const PersistArgs &S, int q) {
                       Comb{S.c0, S.c1, S.c2});
 }
 
-template <int D> ASX_ITEM void fill_item(const PersistArgs &S, const BCSlots &F, int q) {
-  const BatchList &L = S.bc[D];
+ASX_ITEM void fill_item(const PersistArgs &S, const BCSlots &F, int q) {
+  const BatchList &L = S.bc;
   const int f = q / L.n;
   const BatchRef ref = L.map[q - f * L.n];
   const KPatch &P = S.U[ref.pid];
-  bc_point<D>(P.g[F.slot[f]], F.cent[f], P.n[0], P.n[1], P.n[2], P.ng, S.bc_kind,
-              ref.chunk * 256 + (int)threadIdx.x);
+  bc_point(P.g[F.slot[f]], F.cent[f], P.n, P.ng, S.bc_kind, ref.chunk);
 }
 
 // con2prim's primary solve on one chunk of 256 interior zones; failures
@@ -114,10 +113,9 @@ ASX_ITEM void c2p_rest_item(const PersistArgs &S, int z) {
   store_zone(P, off(P, 0, i, j, k), o);
 }
 
-template <int D>
-ASX_DEV void fill_axis(const PersistArgs &S, const BCSlots &F) {
-  const XcdRun r = xcd_run(S.bc[D].n * F.nf);
-  for (int it = r.first; it < r.end; it += r.step) fill_item<D>(S, F, it);
+ASX_DEV void fill_ghosts(const PersistArgs &S, const BCSlots &F) {
+  const XcdRun r = xcd_run(S.bc.n * F.nf);
+  for (int it = r.first; it < r.end; it += r.step) fill_item(S, F, it);
 }
 
 // Register budget: 2 waves per SIMD (256 VGPRs), what the con2prim solve
@@ -151,11 +149,7 @@ void k_stage_persist(const PersistArgs *__restrict__ SA) {
   }
   phase_barrier(grid);
   // 3. fill of the evolved fields
-  fill_axis<0>(S, S.state);
-  phase_barrier(grid);
-  fill_axis<1>(S, S.state);
-  phase_barrier(grid);
-  fill_axis<2>(S, S.state);
+  fill_ghosts(S, S.state);
   phase_barrier(grid);
   // 4. con2prim, primary solver
   {
@@ -172,11 +166,7 @@ void k_stage_persist(const PersistArgs *__restrict__ SA) {
   }
   phase_barrier(grid);
   // 6. fill of the synced primitives
-  fill_axis<0>(S, S.prims);
-  phase_barrier(grid);
-  fill_axis<1>(S, S.prims);
-  phase_barrier(grid);
-  fill_axis<2>(S, S.prims);
+  fill_ghosts(S, S.prims);
 }
 
 // ---------------------------------------------------------------------------

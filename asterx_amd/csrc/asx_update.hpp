@@ -386,63 +386,71 @@ ASX_DEV double psi_rhs(const KPatch &P, int i, int j, int k, const RhsArgs &A) {
   return -dF - A.lorenz_damp_fac * P.g[ASX_ALP][ov] * P.g[ASX_PSI][ov];
 }
 
-// The same fill for up to kMaxBC grid functions of any centering in one
-// launch per axis (blockIdx.y = grid function): one work-item per ghost point,
-// point t of the 2 ng ghost layers normal to D (x fastest, so that the layers
-// normal to y and z are written in full rows).  Each ghost value depends
-// only on interior points along D, so the points of one axis are
-// independent; the axes run in order x, y, z as in k_bc.
-template <int D>
-ASX_DEV void bc_point(double *g, int c, int n0, int n1, int n2, int ng, int kind, int t) {
-  const int n[3] = {n0, n1, n2};
-  const int e[3] = {n0 + 2 * ng + (c & 1), n1 + 2 * ng + ((c >> 1) & 1),
-                    n2 + 2 * ng + ((c >> 2) & 1)};
-  // The axes run in the order x, y, z, and each pass reads only interior
-  // rows / planes along its own axis, so the x pass covers the interior rows
-  // in y and z and the y pass the interior planes in z: the ghost rows and
-  // planes of a later axis are written by that axis's pass.  (Covering them
-  // too, as a single pass per axis over the full extent would, only writes
-  // values the later pass overwrites.)
-  int w[3] = {e[0], e[1], e[2]}, o[3] = {0, 0, 0};
-#pragma unroll
-  for (int a = D + 1; a < 3; ++a) {
-    w[a] = e[a] - 2 * ng;
-    o[a] = ng;
-  }
-  w[D] = 2 * ng;
-  if (t >= w[0] * w[1] * w[2]) return;
-  int x[3] = {t % w[0] + o[0], (t / w[0]) % w[1] + o[1], t / (w[0] * w[1]) + o[2]};
-  const int lo = ng, hi = ng + n[D] - 1 + ((c >> D) & 1);
-  const int q = x[D] < ng ? x[D] : hi + 1 + (x[D] - ng);
-  const int64_t ex = e[0], exy = (int64_t)e[0] * e[1];
-  const int64_t sd = D == 0 ? 1 : (D == 1 ? ex : exy);
-  x[D] = 0;
-  double *l = g + x[0] + x[1] * ex + x[2] * exy;
-  double v;
-  if (q < lo) {
-    if (kind == ASX_BC_LINEAR)
-      v = l[lo * sd] + (lo - q) * (l[lo * sd] - l[(lo + 1) * sd]);
-    else if (kind == ASX_BC_PERIODIC)
-      v = l[(q + n[D]) * sd];
-    else
-      v = l[lo * sd];
-  } else {
-    if (kind == ASX_BC_LINEAR)
-      v = l[hi * sd] + (q - hi) * (l[hi * sd] - l[(hi - 1) * sd]);
-    else if (kind == ASX_BC_PERIODIC)
-      v = l[(q - n[D]) * sd];
-    else
-      v = l[hi * sd];
-  }
-  l[q * sd] = v;
+// Boundary fill of one ghost point.  The reference fills axis by axis, x,
+// then y, then z, each over the ghosts of the axes before it, so a ghost
+// value is a function of interior points alone: the fills nested in that
+// order.  Evaluated that way (the same operations on the same values, so the
+// same bits) no ghost point reads another one, and one launch fills every
+// axis of every grid function.  Copy and periodic fills read one interior
+// point, the linear one two per axis the point is outside of (at most 8).
+struct BCAxis {
+  int s, d, m; // sources along the axis: s, and s + d when m > 0 (linear)
+};
+ASX_DEV BCAxis bc_axis(int q, int lo, int hi, int n, int kind) {
+  const bool below = q < lo;
+  if (!below && q <= hi) return BCAxis{q, 0, 0};
+  if (kind == ASX_BC_PERIODIC) return BCAxis{below ? q + n : q - n, 0, 0};
+  if (kind == ASX_BC_LINEAR)
+    return below ? BCAxis{lo, 1, lo - q} : BCAxis{hi, -1, q - hi};
+  return BCAxis{below ? lo : hi, 0, 0};
 }
-// points of bc_point's pass normal to d for the widest centering (vertex on
-// every axis): the full extent on the axes before d, the interior after it
-__host__ inline int bc_points(const int n[3], int ng, int d) {
-  int w[3] = {n[0] + 2 * ng + 1, n[1] + 2 * ng + 1, n[2] + 2 * ng + 1};
-  for (int a = d + 1; a < 3; ++a) w[a] = n[a] + 1;
-  w[d] = 2 * ng;
-  return w[0] * w[1] * w[2];
+// v at l, extrapolated over the axes 0..D
+template <int D>
+ASX_DEV double bc_value(const double *l, const BCAxis (&a)[3], const int64_t (&st)[3]) {
+  if constexpr (D < 0) {
+    return *l;
+  } else {
+    l += a[D].s * st[D];
+    const double v = bc_value<D - 1>(l, a, st);
+    if (a[D].m == 0) return v;
+    return v + a[D].m * (v - bc_value<D - 1>(l + a[D].d * st[D], a, st));
+  }
+}
+// Ghost point of work-item threadIdx.x of workgroup b (x fastest, so that the
+// layers normal to y and z are written in full rows) of a grid function of
+// centering c.
+ASX_DEV void bc_point(double *g, int c, const int (&n)[3], int ng, int kind, int b) {
+  int d = 0, nb = bc_blocks(n, ng, 0);
+  if (b >= nb) {
+    b -= nb;
+    d = 1;
+    nb = bc_blocks(n, ng, 1);
+    if (b >= nb) {
+      b -= nb;
+      d = 2;
+    }
+  }
+  const int t = b * 256 + (int)threadIdx.x;
+  const int e[3] = {n[0] + 2 * ng + (c & 1), n[1] + 2 * ng + ((c >> 1) & 1),
+                    n[2] + 2 * ng + ((c >> 2) & 1)};
+  int w[3], o[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    w[a] = a < d ? e[a] : (a == d ? 2 * ng : e[a] - 2 * ng);
+    o[a] = a > d ? ng : 0;
+  }
+  if (t >= w[0] * w[1] * w[2]) return;
+  const int r = t / w[0], z = r / w[1];
+  int x[3] = {t - r * w[0] + o[0], r - z * w[1] + o[1], z + o[2]};
+  const int64_t st[3] = {1, e[0], (int64_t)e[0] * e[1]};
+  BCAxis ax[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int hi = e[a] - ng - 1;
+    if (a == d && x[a] >= ng) x[a] += hi + 1 - ng; // the layers above the interior
+    ax[a] = bc_axis(x[a], ng, hi, n[a], kind);
+  }
+  g[x[0] + x[1] * st[1] + x[2] * st[2]] = bc_value<2>(g, ax, st);
 }
 
 // ---------------------------------------------------------------------------
