@@ -424,6 +424,30 @@ void set_variant(int kc, int v) {
   it->second[kc] = v;
 }
 
+// The faces of the three directions (boxes b) and the vertex auxiliaries: one
+// launch, or one per direction where the caller has set a launch shape or
+// times the kernel classes.
+asx_status faces(const KPatch &P, FluxArgs A, const Box b[3], int method, hipStream_t s,
+                 bool tab) {
+  int v[3];
+  for (int d = 0; d < 3; ++d) v[d] = variant_of(ASX_KC_FACE_X + d);
+  if (!(v[0] | v[1] | v[2]) && !g_timing.load(std::memory_order_relaxed))
+    return dev_status(launch_faces(P, A, b, method, s, tab));
+  const int aux = A.with_aux;
+  for (int d = 0; d < 3; ++d) {
+    for (int q = 0; q < 3; ++q) {
+      A.lo[q] = b[d].lo[q];
+      A.cnt[q] = b[d].cnt[q];
+    }
+    A.with_aux = d == 2 && aux; // the vertex aux ride on the z-face launch
+    const asx_status st = dev_status(timed(ASX_KC_FACE_X + d, s, [&] {
+      return launch_flux(d, P, A, method, v[d], s, tab);
+    }));
+    if (st) return st;
+  }
+  return ASX_OK;
+}
+
 unsigned long long *counter_buf(int dev) {
   std::lock_guard<std::mutex> lk(g_mu);
   auto it = g_cnt.find(dev);
@@ -813,25 +837,19 @@ asx_status asx_fluxes(const asx_patch *pt, const asx_params *par, int32_t face_h
   A.rec_var = par->recon_type;
   A.with_T = par->reconstruct_with_temperature;
   A.write_uct = uct;
+  A.write_normal = 1;
   A.bstag_from_A = 0; // AsterX_Fluxes reads dB_stag (schedule.ccl:173-194)
   A.cnt_dev = cd;
-  A.with_aux = 0;
+  Box fb[3];
   for (int d = 0; d < 3; ++d) {
     int halo[3] = {face_halo, face_halo, face_halo};
     halo[d] = 0;
-    const Box b = box(pt, 1 << d, halo);
-    for (int q = 0; q < 3; ++q) {
-      A.lo[q] = b.lo[q];
-      A.cnt[q] = b.cnt[q];
-    }
-    if (d == 2 && aux) { // CalcAuxForAvecPsi rides on the z-face launch
-      const int h = 2 * face_halo;
-      const int ha[3] = {h, h, h};
-      A.with_aux = 1;
-      A.aux = box(pt, 7, ha);
-    }
-    if ((st = dev_status(timed(ASX_KC_FACE_X + d, s, [&] { return launch_flux(d, P, A, par->reconstruction_method, variant_of(ASX_KC_FACE_X + d), s, tab); })))) return st;
+    fb[d] = box(pt, 1 << d, halo);
   }
+  const int ha[3] = {2 * face_halo, 2 * face_halo, 2 * face_halo};
+  A.with_aux = aux; // CalcAuxForAvecPsi
+  A.aux = box(pt, 7, ha);
+  if ((st = faces(P, A, fb, par->reconstruction_method, s, tab))) return st;
   if (cnt) {
     unsigned long long hbuf[2];
     if (hipMemcpyAsync(hbuf, cd, sizeof(hbuf), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -1558,28 +1576,23 @@ static asx_status substep_impl(const asx_patch *stage, const asx_state *u0,
   A.rec_var = par->recon_type;
   A.with_T = par->reconstruct_with_temperature;
   A.write_uct = par->use_uct;
+  A.write_normal = 0; // the update reads none of them
   // the faces take their normal field as the curl of the stage's A (what
   // ComputedBstagFromA would store on the interior faces)
   A.bstag_from_A = 1;
   A.cnt_dev = nullptr;
   A.with_aux = 0;
   const int fh = bc ? 0 : 1;
+  Box fb[3];
   for (int d = 0; d < 3; ++d) {
     int halo[3] = {fh, fh, fh};
     halo[d] = 0;
-    const Box b = box(stage, 1 << d, halo);
-    for (int q = 0; q < 3; ++q) {
-      A.lo[q] = b.lo[q];
-      A.cnt[q] = b.cnt[q];
-    }
-    if (d == 2) { // the vertex aux ride on the z-face launch
-      const int h = 2 * fh;
-      const int ha[3] = {h, h, h};
-      A.with_aux = 1;
-      A.aux = box(stage, 7, ha);
-    }
-    if ((st = dev_status(timed(ASX_KC_FACE_X + d, s, [&] { return launch_flux(d, P, A, par->reconstruction_method, variant_of(ASX_KC_FACE_X + d), s, tab); })))) return st;
+    fb[d] = box(stage, 1 << d, halo);
   }
+  const int ha[3] = {2 * fh, 2 * fh, 2 * fh};
+  A.with_aux = 1;
+  A.aux = box(stage, 7, ha);
+  if ((st = faces(P, A, fb, par->reconstruction_method, s, tab))) return st;
   if (bc) {
     BCList L;
     L.nf = 0;
@@ -1590,7 +1603,11 @@ static asx_status substep_impl(const asx_patch *stage, const asx_state *u0,
         ++L.nf;
       }
     };
-    add(ASX_FXDENS, ASX_FZBZ);
+    for (int d = 0; d < 3; ++d) { // but for the normal field's flux
+      const int f = ASX_FXDENS + 10 * d;
+      add(f, f + 6 + d);
+      add(f + 8 + d, f + 9);
+    }
     add(ASX_FX, ASX_G);
     if (par->use_uct) {
       // dB_stag on the interior faces (AsterX_ComputedBstagFromA), SYNCed
@@ -1707,6 +1724,31 @@ asx_status asx_autotune_substep(const asx_patch *stage, const asx_state *u0,
     }
   }
   for (int q = 0; q < 4; ++q) set_variant(tuned[q], arg[q]);
+  // the faces in one launch (every face class at its default) or one launch
+  // per direction in the shapes just found: the shorter substep
+  if (!st && (arg[0] | arg[1] | arg[2])) {
+    hipStream_t s = (hipStream_t)stream;
+    float ms[2] = {0, 0};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    if (hipEventCreate(&ev[0]) != hipSuccess || hipEventCreate(&ev[1]) != hipSuccess)
+      st = ASX_ERR_DEVICE;
+    if (!st) st = asx_timing_enable(0);
+    for (int one = 0; one < 2 && !st; ++one) {
+      for (int q = 0; q < 3; ++q) set_variant(tuned[q], one ? 0 : arg[q]);
+      if ((st = asx_substep(stage, u0, out, c0, c1, c2, par, stream))) break;
+      if (hipEventRecord(ev[0], s) != hipSuccess) st = ASX_ERR_DEVICE;
+      for (int r = 0; r < reps && !st; ++r)
+        st = asx_substep(stage, u0, out, c0, c1, c2, par, stream);
+      if (!st && (hipEventRecord(ev[1], s) != hipSuccess ||
+                  hipEventSynchronize(ev[1]) != hipSuccess ||
+                  hipEventElapsedTime(&ms[one], ev[0], ev[1]) != hipSuccess))
+        st = ASX_ERR_DEVICE;
+    }
+    if (st || ms[0] < ms[1])
+      for (int q = 0; q < 3; ++q) set_variant(tuned[q], arg[q]);
+    for (hipEvent_t x : ev)
+      if (x) (void)hipEventDestroy(x);
+  }
   {
     std::lock_guard<std::mutex> l(g_tmu);
     asx_status st2 = drain_timing();
@@ -2176,6 +2218,7 @@ FluxArgs plan_flux_args(const asx_params *par) {
   A.rec_var = par->recon_type;
   A.with_T = par->reconstruct_with_temperature;
   A.write_uct = 0;
+  A.write_normal = 0;
   A.bstag_from_A = 1; // the faces take the curl of the stage's A
   A.cnt_dev = nullptr;
   for (int q = 0; q < 3; ++q) A.lo[q] = A.cnt[q] = 0;
@@ -2186,6 +2229,10 @@ FluxArgs plan_flux_args(const asx_params *par) {
 
 // Stage-s stencil work: faces (normal field from A), aux, update into
 // buffer (1,2,0)[s].
+int plan_face_shape(const asx_batch *b, int d) {
+  return b->var[d] ? b->var[d] : face_shape(d, b->par.reconstruction_method, false);
+}
+
 asx_status plan_stencil(asx_batch *b, int s, hipStream_t str) {
   const int bi = kStageIn[s], bo = kStageOut[s];
   const KPatch *T = b->stab[bi];
@@ -2193,7 +2240,7 @@ asx_status plan_stencil(asx_batch *b, int s, hipStream_t str) {
   asx_status st;
   const FluxArgs A = plan_flux_args(&b->par);
   for (int d = 0; d < 3; ++d) {
-    const int v = b->var[d];
+    const int v = plan_face_shape(b, d);
     if ((st = plan_launch(b, BK_FACE + d, v, &L))) return st;
     if ((st = dev_status(timed(ASX_KC_FACE_X + d, str, [&] {
            return launch_face_batch(d, T, A, L->box, L->map, L->nmap,
@@ -2267,7 +2314,7 @@ asx_status plan_prepare(asx_batch *b) {
   asx_status st;
   for (int k = 0; k < BK_COUNT; ++k) {
     int v = 0;
-    if (k >= BK_FACE && k < BK_FACE + 3) v = b->var[k - BK_FACE];
+    if (k >= BK_FACE && k < BK_FACE + 3) v = plan_face_shape(b, k - BK_FACE);
     if (k == BK_UPDATE) v = b->var[3];
     if ((st = plan_launch(b, k, v, &L))) return st;
   }

@@ -63,8 +63,7 @@ ASX_DEV void cell_recon_s(const double s[5], const double ps[5], const double vs
   } else if (M == ASX_RECON_WENOZ) {
     wenoz_cell(s[0], s[1], s[2], s[3], s[4], rp.weno_eps, lo, up);
   } else {
-    up = mp5_side(s[0], s[1], s[2], s[3], s[4], rp.mp5_alpha);
-    lo = mp5_side(s[4], s[3], s[2], s[1], s[0], rp.mp5_alpha);
+    mp5_cell(s[0], s[1], s[2], s[3], s[4], rp.mp5_alpha, lo, up);
   }
 }
 template <int M>
@@ -129,12 +128,23 @@ ASX_DEV void recon_cell(const KPatch &P, const FluxArgs &A, int oc, Side &lo, Si
 #pragma unroll
   for (int q = 0; q < kSideVars; ++q) cell_stencil<M>(P.g[slot[q]], oc, sc, st[q]);
   mid();
+  // one variable's temporaries at a time (no instruction; the compiler would
+  // take the differences of several variables together, and spill)
+  auto in_order = [](double (&s)[5]) {
+    constexpr int m0 = StencilSpan<M>::m0;
+#pragma unroll
+    for (int m = m0; m <= 4 - m0; ++m) asm volatile("" : "+v"(s[m]));
+  };
   double *const lv[kSideVars] = {&lo.rho, &lo.ent, &lo.ye, &lo.th, &lo.b1,
                                  &lo.b2, &lo.v[0], &lo.v[1], &lo.v[2]};
   double *const uv[kSideVars] = {&up.rho, &up.ent, &up.ye, &up.th, &up.b1,
                                  &up.b2, &up.v[0], &up.v[1], &up.v[2]};
 #pragma unroll
-  for (int q = 0; q < 4; ++q) cell_recon_s<M>(st[q], ps, vs, q == 0, A.rp, *lv[q], *uv[q]);
+  for (int q = 0; q < 4; ++q) {
+    in_order(st[q]);
+    cell_recon_s<M>(st[q], ps, vs, q == 0, A.rp, *lv[q], *uv[q]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   flo = (lo.rho <= 0.0) || (lo.ent <= 0.0) || (lo.ye <= 0.0) || (lo.th <= 0.0);
   fup = (up.rho <= 0.0) || (up.ent <= 0.0) || (up.ye <= 0.0) || (up.th <= 0.0);
   const bool any = flo || fup;
@@ -153,8 +163,10 @@ ASX_DEV void recon_cell(const KPatch &P, const FluxArgs &A, int oc, Side &lo, Si
   for (int q = 0; q < 4; ++q) fix(q);
 #pragma unroll
   for (int q = 4; q < kSideVars; ++q) {
+    in_order(st[q]);
     cell_recon_s<M>(st[q], ps, vs, false, A.rp, *lv[q], *uv[q]);
     fix(q);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -373,8 +385,9 @@ ASX_DEV void face_flux(const KPatch &P, const FluxArgs &A, int i, int j, int k,
     if constexpr (TAB) {
       cs2[f] = cs2t[f];
     } else {
-      const double cs = eos.csnd(eps[f]);
-      cs2[f] = cs * cs;
+      // the square itself (NaN, as the sound speed would be, below zero)
+      const double c2 = eos.csnd2(eps[f]);
+      cs2[f] = c2 >= 0.0 ? c2 : __builtin_nan("");
     }
     h[f] = 1 + eps[f] + press[f] * irho[f];
     dens[f] = sqrtg * rho[f] * W[f];
@@ -453,7 +466,8 @@ ASX_DEV void face_flux(const KPatch &P, const FluxArgs &A, int i, int j, int k,
     double fb[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) fb[f] = uj * E[ck][f] - uk * E[cj][f];
-    F[7 + c][ofc] = (D != c) * num(Bt[c][0], Bt[c][1], fb[0], fb[1]);
+    if (c != D || A.write_normal)
+      F[7 + c][ofc] = (D != c) * num(Bt[c][0], Bt[c][1], fb[0], fb[1]);
   }
 
   if (A.write_uct) { // fluxes.cxx:776-793

@@ -31,6 +31,78 @@ void k_face(KPatch P, FluxArgs A, int ntx, int nty, int ntz) {
   }
 }
 
+// Tile shapes used where the caller has set none.  Staging the metric pays
+// where the reconstruction's registers leave room for it beside the stencils
+// (192^3 substep, x and z staged against neither: WENO-Z 3.33 / 3.45 ms, PPM
+// 3.73 / 3.52; table 100 x 90 x 80, PPM: 0.555 / 0.584); in y, whose staged
+// tiles are narrow, the 16 x 16 rows of per-face loads are as fast.
+template <int M, bool TAB> struct FaceShapes {
+  static constexpr bool staged = TAB || M == ASX_RECON_WENOZ || M == ASX_RECON_MP5;
+  static constexpr int X = staged ? 5 : 4, Y = 0, Z = staged ? 5 : 3;
+};
+int face_shape(int d, int method, bool tab) {
+  using S = FaceShapes<ASX_RECON_WENOZ, false>;
+  using U = FaceShapes<ASX_RECON_PPM, false>;
+  const bool staged = tab || method == ASX_RECON_WENOZ || method == ASX_RECON_MP5;
+  return d == 0 ? (staged ? S::X : U::X) : d == 1 ? S::Y : (staged ? S::Z : U::Z);
+}
+
+// Faces of the three directions and, where they are asked for, the vertex
+// auxiliaries in one launch.  On a small patch the three directions' latencies
+// overlap (22 x 17 x 13: 40 us as three launches, 10 as one); on a large one
+// the auxiliaries, bound by memory, run beside the faces' arithmetic, and the
+// last, partly filled waves of two launches go (192^3: 2.15 -> 1.98 ms).
+// The tiles are visited in chunks: per[q] tiles of kind q (x, y, z faces,
+// auxiliaries) from the same part of the patch, then the next chunk.
+struct FaceSet {
+  int lo[3][3], cnt[3][3], nt[3][2];
+  int n[4], per[4], group; // tiles, tiles per chunk, sum of per
+};
+template <int M, int VX, int VY, int VZ, bool TAB>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(TAB ? ASX_FACE_WAVES_TAB : ASX_FACE_WAVES)))
+void k_faces(KPatch P, FluxArgs A, FaceSet F) {
+  __shared__ FaceLDS S;
+  using MX = MetricBox<0, VX>;
+  using MY = MetricBox<1, VY>;
+  using MZ = MetricBox<2, VZ>;
+  constexpr int NX = MX::ok ? MX::N : 1, NY = MY::ok ? MY::N : 1, NZ = MZ::ok ? MZ::N : 1;
+  __shared__ double MS[NX > NY ? (NX > NZ ? NX : NZ) : (NY > NZ ? NY : NZ)];
+  const int u = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  const int c = u / F.group;
+  int r = u - c * F.group;
+  if (r < F.per[0]) {
+    const int b = c * F.per[0] + r;
+    if (b < F.n[0])
+      face_tile<0, M, VX, TAB>(P, A, F.lo[0], F.cnt[0], b, F.nt[0][0], F.nt[0][1], S,
+                               MX::ok ? MS : nullptr);
+    return;
+  }
+  r -= F.per[0];
+  if (r < F.per[1]) {
+    const int b = c * F.per[1] + r;
+    if (b < F.n[1])
+      face_tile<1, M, VY, TAB>(P, A, F.lo[1], F.cnt[1], b, F.nt[1][0], F.nt[1][1], S,
+                               MY::ok ? MS : nullptr);
+    return;
+  }
+  r -= F.per[1];
+  if (r < F.per[2]) {
+    const int b = c * F.per[2] + r;
+    if (b < F.n[2])
+      face_tile<2, M, VZ, TAB>(P, A, F.lo[2], F.cnt[2], b, F.nt[2][0], F.nt[2][1], S,
+                               MZ::ok ? MS : nullptr);
+    return;
+  }
+  r -= F.per[2];
+  const int64_t t = ((int64_t)c * F.per[3] + r) * 256 + threadIdx.x;
+  if (t < A.aux.total()) {
+    int i, j, k;
+    A.aux.ijk(t, i, j, k);
+    aux_point(P, i, j, k);
+  }
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void k_bstag(KPatch P, Box B, double *out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -140,7 +212,7 @@ static hipError_t launch_flux_dv(const KPatch &P, const FluxArgs &A, int method,
 template <int D>
 static hipError_t launch_flux_d(const KPatch &P, const FluxArgs &A, int method, int variant,
                                 hipStream_t s, bool tab) {
-  switch (variant) {
+  switch (variant ? variant : face_shape(D, method, tab)) {
   case 1: return launch_flux_dv<D, 1>(P, A, method, s, tab);
   case 2: return launch_flux_dv<D, 2>(P, A, method, s, tab);
   case 3: return launch_flux_dv<D, 3>(P, A, method, s, tab);
@@ -148,8 +220,69 @@ static hipError_t launch_flux_d(const KPatch &P, const FluxArgs &A, int method, 
   case 5: return launch_flux_dv<D, 5>(P, A, method, s, tab);
   case 6: return launch_flux_dv<D, 6>(P, A, method, s, tab);
   case 7: return launch_flux_dv<D, 7>(P, A, method, s, tab);
-  default: return launch_flux_dv<D, 0>(P, A, method, s, tab);
+  default: return launch_flux_dv<D, D == 1 ? 0 : 5>(P, A, method, s, tab);
   }
+}
+
+template <int D, int V> static void face_set(FaceSet &F, const Box &b) {
+  using T = FaceTile<D, V>;
+  const int ex[3] = {T::X, T::Y, T::Z};
+  int nt[3];
+  for (int q = 0; q < 3; ++q) {
+    const int per = q == D ? ex[q] - 1 : ex[q];
+    F.lo[D][q] = b.lo[q];
+    F.cnt[D][q] = b.cnt[q];
+    nt[q] = (b.cnt[q] + per - 1) / per;
+  }
+  F.nt[D][0] = nt[0];
+  F.nt[D][1] = nt[1];
+  F.n[D] = nt[0] * nt[1] * nt[2];
+}
+template <int M, int VX, int VY, int VZ, bool TAB>
+static void launch_faces_v(const KPatch &P, const FluxArgs &A, const Box b[3], hipStream_t s) {
+  FaceSet F;
+  face_set<0, VX>(F, b[0]);
+  face_set<1, VY>(F, b[1]);
+  face_set<2, VZ>(F, b[2]);
+  F.n[3] = A.with_aux ? (int)((A.aux.htotal() + 255) / 256) : 0;
+  // Chunks of up to 256 tiles of a kind (192^3 faces and auxiliaries, WENO-Z:
+  // 2.07 ms with 64 and 1.98 with 256 or 512 tiles, 2.21 as one launch per
+  // direction), whole chunks per XCD (the kinds differ in cost).
+  const int most = std::max(F.n[0], std::max(F.n[1], F.n[2]));
+  const int chunks = most < 64 ? 1 : 8 * std::max(1, most / (8 * 256));
+  F.group = 0;
+  for (int q = 0; q < 4; ++q) {
+    F.per[q] = (F.n[q] + chunks - 1) / chunks;
+    F.group += F.per[q];
+  }
+  hipLaunchKernelGGL((k_faces<M, VX, VY, VZ, TAB>), dim3((unsigned)(chunks * F.group)),
+                     dim3(256), 0, s, P, A, F);
+}
+template <int M, bool TAB>
+static void launch_faces_m(const KPatch &P, const FluxArgs &A, const Box b[3], hipStream_t s) {
+  using T = FaceShapes<M, TAB>;
+  launch_faces_v<M, T::X, T::Y, T::Z, TAB>(P, A, b, s);
+}
+hipError_t launch_faces(const KPatch &P, const FluxArgs &A, const Box b[3], int method,
+                        hipStream_t s, bool tab) {
+  if (tab) {
+    switch (method) {
+    case ASX_RECON_PPM: launch_faces_m<ASX_RECON_PPM, true>(P, A, b, s); break;
+    case ASX_RECON_WENOZ: launch_faces_m<ASX_RECON_WENOZ, true>(P, A, b, s); break;
+    case ASX_RECON_MP5: launch_faces_m<ASX_RECON_MP5, true>(P, A, b, s); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
+  switch (method) {
+  case ASX_RECON_GODUNOV: launch_faces_m<ASX_RECON_GODUNOV, false>(P, A, b, s); break;
+  case ASX_RECON_MINMOD: launch_faces_m<ASX_RECON_MINMOD, false>(P, A, b, s); break;
+  case ASX_RECON_MONOCENTRAL: launch_faces_m<ASX_RECON_MONOCENTRAL, false>(P, A, b, s); break;
+  case ASX_RECON_PPM: launch_faces_m<ASX_RECON_PPM, false>(P, A, b, s); break;
+  case ASX_RECON_WENOZ: launch_faces_m<ASX_RECON_WENOZ, false>(P, A, b, s); break;
+  default: launch_faces_m<ASX_RECON_MP5, false>(P, A, b, s); break;
+  }
+  return hipGetLastError();
 }
 
 bool flux_tab_method(int method) {
@@ -247,7 +380,7 @@ static void launch_face_batch_d(const KPatch *tab, const FluxArgs &A, const Batc
   case 5: launch_face_batch_dv<D, 5>(tab, A, box, map, nmap, method, s); break;
   case 6: launch_face_batch_dv<D, 6>(tab, A, box, map, nmap, method, s); break;
   case 7: launch_face_batch_dv<D, 7>(tab, A, box, map, nmap, method, s); break;
-  default: launch_face_batch_dv<D, 0>(tab, A, box, map, nmap, method, s); break;
+  default: launch_face_batch_dv<D, D == 1 ? 0 : 5>(tab, A, box, map, nmap, method, s); break;
   }
 }
 

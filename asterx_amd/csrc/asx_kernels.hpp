@@ -113,6 +113,7 @@ struct FluxArgs {
   IdealGas eos;
   TabEOS tab; // used by the table instantiations (evolution_eos = Tabulated3d)
   int lo_method, flux_type, rec_var, with_T, write_uct;
+  int write_normal; // store the (zero) flux of the normal field component
   int bstag_from_A; // normal face field as the curl of A at the face (no dB_stag read)
   int lo[3], cnt[3];
   unsigned long long *cnt_dev; // [nan_faces, lo_faces] or null
@@ -131,9 +132,15 @@ struct StatePtrs {
   double *g[ASX_NUM_STATE];
 };
 
-// tab: the EOS is A.tab (PPM, WENO-Z and MP5 only; reconstruction in T)
+// tab: the EOS is A.tab (PPM, WENO-Z and MP5 only; reconstruction in T);
+// variant: tile shape, 0: face_shape()
 hipError_t launch_flux(int d, const KPatch &P, const FluxArgs &A, int method, int variant,
                        hipStream_t s, bool tab = false);
+// the faces normal to x, y and z over the boxes b[0..2], and the vertex
+// auxiliaries of box A.aux where A.with_aux, in one launch
+hipError_t launch_faces(const KPatch &P, const FluxArgs &A, const Box b[3], int method,
+                        hipStream_t s, bool tab = false);
+int face_shape(int d, int method, bool tab);
 bool flux_tab_method(int method);
 hipError_t launch_bstag(int d, const KPatch &P, const Box &B, double *out,
                         hipStream_t s);

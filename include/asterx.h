@@ -296,7 +296,8 @@ const char *asx_version(void);
 
 /* Kernel timing (diagnostics; no counterpart in the reference).  While
  * enabled, every kernel launch of the library is bracketed by HIP events on
- * the caller's stream.  asx_timing_read returns, for one kernel class, the
+ * the caller's stream, and the faces of one patch run as a launch per
+ * direction, in the same tile shapes.  asx_timing_read returns, for one kernel class, the
  * number of launches and their summed durations in milliseconds since the
  * last asx_timing_enable call, waiting for launches still in flight.
  * Enabling or disabling resets the sums. */
@@ -306,7 +307,7 @@ enum {
   ASX_KC_FACE_Y = 2,
   ASX_KC_FACE_Z = 3,
   ASX_KC_AUX = 4,    /* vertex auxiliaries of the A/Psi gauge (batch plans;
-                        on one patch they ride on the z-face launch) */
+                        on one patch they ride on the face launches) */
   ASX_KC_UPDATE = 5, /* fused RHS + RK combination */
   ASX_KC_C2P = 6,    /* con2prim: every zone, primary solver (patch or batch) */
   ASX_KC_BC = 7,     /* boundary fills */
@@ -354,10 +355,14 @@ asx_status asx_poison_check(const asx_patch *patch, int32_t slot, const int32_t 
  * (up to 52 KB of LDS per workgroup with the face hand-over, three
  * workgroups per CU).  ASX_KC_MLP has two forms of asx_c2p_batch_mlp (network fused
  * into the solver kernel, or a separate forward pass), whose guesses differ
- * by the fp32 summation order only.  The choice is per device (default 0).  asx_autotune_substep
+ * by the fp32 summation order only.  The choice is per device (default 0).
+ * Variant 0 of a face class leaves the shape to the library; while all three
+ * are 0, one launch computes the faces of every direction and the vertex
+ * auxiliaries of a patch.  asx_autotune_substep
  * runs asx_substep with the given arguments once untimed and `reps` times
- * timed for every variant, keeps the fastest per kernel class, and leaves the
- * caller's timing state as it was.  It overwrites `out`. */
+ * timed for every variant, keeps the fastest per kernel class (or the one
+ * launch, where that is faster), and leaves the caller's timing state as it
+ * was.  It overwrites `out`. */
 int32_t asx_variant_count(int32_t kclass);
 asx_status asx_set_variant(int32_t kclass, int32_t v);
 asx_status asx_get_variant(int32_t kclass, int32_t *v);

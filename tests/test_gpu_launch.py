@@ -8,6 +8,7 @@ import pytest
 import oracle
 from asterx_amd import abi
 from asterx_amd.patch import Patch
+from states import make_state
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,32 @@ def test_boundary_fill(n, ng, kind):
         assert np.array_equal(many.numpy(name), h.numpy(name)), name
         assert np.array_equal(one.numpy(name), h.numpy(name)), name
 
+
+@pytest.mark.parametrize("n", [(4, 5, 6), (16, 15, 7), (33, 31, 30)])
+@pytest.mark.parametrize("recon", ["wenoz", "mp5", "ppm", "minmod"])
+@pytest.mark.parametrize("halo", [0, 1])
+def test_faces_in_one_launch(n, recon, halo):
+    """The faces of every direction and the auxiliaries in one launch against
+    one launch per direction in other tile shapes."""
+    torch = _torch()
+    L = _lib()
+    par = abi.params(reconstruction_method=recon, flux_type="HLLE", loworder_method="minmod")
+    names = abi.FLUX + abi.AUX + abi.UCT
+    got = []
+    kcs = [abi.KCLASS["face_" + c] for c in "xyz"]
+    try:
+        for v in (0, 1):
+            for kc in kcs:
+                abi.check("asx_set_variant", L.asx_set_variant(kc, v))
+            d = make_state(n=n, curved=True, zero_entropy_block=True).to("cuda")
+            for name in names:
+                d[name].fill_(0.0)
+            abi.check("asx_fluxes", L.asx_fluxes(C.byref(d.struct()), C.byref(par), halo, None,
+                                                 None))
+            torch.cuda.synchronize()
+            got.append({m: d.numpy(m) for m in names})
+    finally:
+        for kc in kcs:
+            abi.check("asx_set_variant", L.asx_set_variant(kc, 0))
+    for m in names:
+        assert np.array_equal(got[0][m], got[1][m]), m
