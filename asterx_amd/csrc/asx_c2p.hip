@@ -2,6 +2,8 @@
 // with ComputedBstagFromA + ComputedBFromdBstag) and Con2PrimFactory solves
 // on independent zones.  One work-item per cell; flag and iteration
 // histograms are reduced in LDS per block before one atomic per bin.
+#include <algorithm>
+
 #include "asx_zone.hpp"
 
 namespace asx {
@@ -24,15 +26,14 @@ ASX_DEV void hist_flush(HistLDS &h, unsigned long long *g) {
   }
 }
 
-// Pass 1: every zone through the primary solver (compiled for PRIME only,
-// so the backup solvers cost no registers here).  Zones whose primary solve
-// fails store nothing; a wavefront ballot packs their indices into `queue`
-// with one atomic per wavefront.
-template <bool FROM_A, int PRIME, class E>
+// Pass 1: every zone through the primary solver (Palenzuela, the only one a
+// table takes; compiled alone, so the backup costs no registers here).  Zones
+// whose primary solve fails store nothing; a wavefront ballot packs their
+// indices into `queue` with one atomic per wavefront.
+template <bool FROM_A, class E>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(c2p_waves<E>())))
-void k_c2p_main(KPatch P, Box B, E eos, C2PArgs a,
-                                                  unsigned long long *hist, int *queue,
-                                                  unsigned *qcount) {
+void k_c2p_main(KPatch P, Box B, E eos, C2PArgs a, unsigned long long *hist, int *queue,
+                unsigned *qcount) {
   __shared__ HistLDS h;
   if (hist) {
     hist_init(h);
@@ -47,7 +48,7 @@ void k_c2p_main(KPatch P, Box B, E eos, C2PArgs a,
     C2PIn in;
     load_zone<FROM_A>(P, i, j, k, a, in);
     C2POut o;
-    if (con2prim_zone<PRIME>(eos, a, in, o)) {
+    if (con2prim_zone<ASX_C2P_PALENZUELA>(eos, a, in, o)) {
       store_zone(P, off(P, 0, i, j, k), o);
       if (hist) {
         atomicAdd(&h.flags[(int)o.flag], 1u);
@@ -96,53 +97,117 @@ __global__ __launch_bounds__(256) void k_c2p_rest(KPatch P, Box B, E eos, C2PArg
   }
 }
 
-__global__ void k_zero_u32(unsigned *p) { *p = 0u; }
-
-template <int PRIME>
-__global__ __launch_bounds__(256) void k_c2p_main_batch(const KPatch *__restrict__ tab,
-                                                        const int *__restrict__ zbase,
-                                                        IdealGas eos, C2PArgs a,
-                                                        const BatchRef *__restrict__ map,
-                                                        int nmap, int *queue,
-                                                        unsigned *qcount) {
-  const BatchRef r = map[xcd_tile((int)blockIdx.x, nmap)];
-  const KPatch &P = tab[r.pid];
-  const int t = r.chunk * 256 + (int)threadIdx.x;
-  bool fail = false;
-  if (t < P.n[0] * P.n[1] * P.n[2]) {
-    int i, j, k;
-    interior_ijk(P, t, i, j, k);
-    C2PIn in;
-    load_zone<true>(P, i, j, k, a, in);
-    C2POut o;
-    if (con2prim_zone<PRIME>(eos, a, in, o)) store_zone(P, off(P, 0, i, j, k), o);
-    else fail = true;
+// Every zone through the full chain: a zone whose primary fails goes on to
+// the backup in its own lane.  Bound by memory on the ideal gas (60 fields a
+// zone), whose full chain fits the two wavefronts per SIMD that the primary
+// alone takes; so the backup costs the wavefronts that hold a failed zone, and
+// on a patch those are few: they lie together, at a shock or the edge of the
+// atmosphere.  A second pass over queued zones repeats the failed primary in
+// a few wavefronts (253 x 231 x 246 torus, MP5, after 70 substeps: 11.6 ms a
+// substep with the queue, 8.73 so; 64^3 WENO-Z 0.219 -> 0.192 ms; 22 x 17 x 13
+// con2prim 50 -> 26 us; 192^3, no failed zones: the same).
+template <bool FROM_A, class E>
+__global__ __launch_bounds__(256) void k_c2p_one(KPatch P, Box B, E eos, C2PArgs a,
+                                                 unsigned long long *hist) {
+  __shared__ HistLDS h;
+  if (hist) {
+    hist_init(h);
+    __syncthreads();
   }
-  queue_push(fail, zbase[r.pid] + t, queue, qcount);
-}
-
-__global__ __launch_bounds__(256) void k_c2p_rest_batch(const KPatch *__restrict__ tab,
-                                                        const int *__restrict__ zbase, int np,
-                                                        IdealGas eos, C2PArgs a,
-                                                        const int *queue,
-                                                        const unsigned *qcount) {
-  const unsigned nq = *qcount;
-  for (unsigned q = blockIdx.x * blockDim.x + threadIdx.x; q < nq;
-       q += gridDim.x * blockDim.x) {
-    const int z = queue[q];
-    const int p = patch_of(zbase, np, z);
-    const KPatch &P = tab[p];
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < B.total()) {
     int i, j, k;
-    interior_ijk(P, z - zbase[p], i, j, k);
+    B.ijk(t, i, j, k);
     C2PIn in;
-    load_zone<true>(P, i, j, k, a, in);
+    load_zone<FROM_A>(P, i, j, k, a, in);
     C2POut o;
     con2prim_cell(eos, a, in, o);
     store_zone(P, off(P, 0, i, j, k), o);
+    if (hist) {
+      atomicAdd(&h.flags[(int)o.flag], 1u);
+      atomicAdd(&h.iters[o.iters < 63 ? o.iters : 63], 1u);
+    }
+  }
+  if (hist) {
+    __syncthreads();
+    hist_flush(h, hist);
   }
 }
 
-// Independent zones (layout of asx_c2p_batch in include/asterx.h).
+__global__ void k_zero_u32(unsigned *p) { *p = 0u; }
+
+// k_c2p_one over the patches of a batch
+__global__ __launch_bounds__(256) void k_c2p_patches(const KPatch *__restrict__ tab, IdealGas eos,
+                                                     C2PArgs a, const BatchRef *__restrict__ map,
+                                                     int nmap) {
+  const BatchRef r = map[xcd_tile((int)blockIdx.x, nmap)];
+  const KPatch &P = tab[r.pid];
+  const int t = r.chunk * 256 + (int)threadIdx.x;
+  if (t >= P.n[0] * P.n[1] * P.n[2]) return;
+  int i, j, k;
+  interior_ijk(P, t, i, j, k);
+  C2PIn in;
+  load_zone<true>(P, i, j, k, a, in);
+  C2POut o;
+  con2prim_cell(eos, a, in, o);
+  store_zone(P, off(P, 0, i, j, k), o);
+}
+
+// Independent zones (layout of asx_c2p_batch in include/asterx.h) in two
+// passes without scratch memory: every zone through the primary solver, which
+// alone sets the register budget (152 VGPRs and 3 waves per SIMD for Noble,
+// 208 and 2 for the full chain); a zone it fails gets the flag kZoneFailed,
+// which the second pass looks for.  Bound by the latency of the Newton
+// steps' dependent square roots and reciprocals: 4 000 037 zones from the
+// previous step's primitives 0.770 -> 0.497 ms (0.13 of them the second pass).
+constexpr double kZoneFailed = -1.0;
+template <int PRIME>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+void k_c2p_zones(int64_t nz, const double *cons, const double *g, const double *seed,
+                 double *prim, double *flag, int32_t *iters, IdealGas eos, C2PArgs a) {
+  const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (z >= nz) return;
+  C2PIn in;
+  batch_zone_in(z, nz, cons, g, seed, a, in);
+  C2POut o;
+  if (con2prim_zone<PRIME>(eos, a, in, o)) {
+    batch_zone_out(z, nz, o, prim, flag);
+    iters[z] = o.iters;
+  } else {
+    flag[z] = kZoneFailed;
+  }
+}
+// The failed zones among each wavefront's `per` <= kRestZones, gathered in LDS, through
+// the full chain: a chain of thirty failed Newton steps and the backup's
+// iterations, so what counts is that the few zones spread over all SIMDs
+// (4 000 037 zones: 0.19 ms with workgroups of 256 for 4096 zones, 0.13 with
+// a wavefront each).
+constexpr int kRestZones = 4096;
+__global__ __launch_bounds__(64)
+void k_c2p_zones_rest(int64_t nz, int per, const double *cons, const double *g,
+                      const double *seed, double *prim, double *flag, int32_t *iters,
+                      IdealGas eos, C2PArgs a) {
+  __shared__ int list[kRestZones];
+  __shared__ int n;
+  if (threadIdx.x == 0) n = 0;
+  __syncthreads();
+  const int64_t z0 = (int64_t)blockIdx.x * per;
+#pragma unroll 16
+  for (int q = threadIdx.x; q < per; q += 64)
+    if (z0 + q < nz && flag[z0 + q] == kZoneFailed) list[atomicAdd(&n, 1)] = q;
+  __syncthreads();
+  const int nq = n;
+  for (int q = threadIdx.x; q < nq; q += 64) {
+    const int64_t z = z0 + list[q];
+    C2PIn in;
+    batch_zone_in(z, nz, cons, g, seed, a, in);
+    C2POut o;
+    con2prim_cell(eos, a, in, o);
+    batch_zone_out(z, nz, o, prim, flag);
+    iters[z] = o.iters;
+  }
+}
+// In one pass, for few zones.
 __global__ __launch_bounds__(256) void k_c2p_batch(int64_t nz, const double *cons,
                                                    const double *g, const double *seed,
                                                    double *prim, double *flag,
@@ -158,6 +223,13 @@ __global__ __launch_bounds__(256) void k_c2p_batch(int64_t nz, const double *con
   iters[z] = o.iters;
 }
 
+template <class E>
+static void c2p_one_t(const KPatch &P, const Box &b, const E &eos, const C2PArgs &a,
+                      bool from_A, unsigned long long *hist, hipStream_t s) {
+  if (from_A) hipLaunchKernelGGL((k_c2p_one<true, E>), b.grid(), dim3(256), 0, s, P, b, eos, a, hist);
+  else hipLaunchKernelGGL((k_c2p_one<false, E>), b.grid(), dim3(256), 0, s, P, b, eos, a, hist);
+}
+
 static Box c2p_box(const KPatch &P) {
   Box b;
   for (int d = 0; d < 3; ++d) {
@@ -167,95 +239,45 @@ static Box c2p_box(const KPatch &P) {
   return b;
 }
 
-template <bool FROM_A, int PRIME, class E>
-static void c2p_main_t(const KPatch &P, const Box &b, const E &eos, const C2PArgs &a,
-                       unsigned long long *hist, int *queue, unsigned *qcount, hipStream_t s) {
-  hipLaunchKernelGGL((k_c2p_main<FROM_A, PRIME, E>), b.grid(), dim3(256), 0, s, P, b, eos, a,
-                     hist, queue, qcount);
-}
-template <class E>
-static void c2p_rest_t(const KPatch &P, const Box &b, const E &eos, const C2PArgs &a,
-                       bool from_A, unsigned long long *hist, const int *queue,
-                       const unsigned *qcount, hipStream_t s) {
-  const int64_t nz = b.htotal();
-  // enough work-items for a few percent of the zones; more stride
-  const unsigned g2 = (unsigned)((nz + 255) / 256 < 2048 ? (nz + 255) / 256 : 2048);
-  if (from_A)
-    hipLaunchKernelGGL((k_c2p_rest<true, E>), dim3(g2), dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
-  else
-    hipLaunchKernelGGL((k_c2p_rest<false, E>), dim3(g2), dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
-}
-
-hipError_t launch_con2prim_main(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
-                                bool from_A, unsigned long long *hist, int *queue,
-                                unsigned *qcount, hipStream_t s) {
-  const Box b = c2p_box(P);
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, qcount);
-  if (b.htotal() <= 0) return hipGetLastError();
-  const int pr = a.prime;
-  if (from_A) {
-    if (pr == ASX_C2P_NOBLE) c2p_main_t<true, ASX_C2P_NOBLE>(P, b, eos, a, hist, queue, qcount, s);
-    else if (pr == ASX_C2P_ENTROPY) c2p_main_t<true, ASX_C2P_ENTROPY>(P, b, eos, a, hist, queue, qcount, s);
-    else c2p_main_t<true, ASX_C2P_PALENZUELA>(P, b, eos, a, hist, queue, qcount, s);
-  } else {
-    if (pr == ASX_C2P_NOBLE) c2p_main_t<false, ASX_C2P_NOBLE>(P, b, eos, a, hist, queue, qcount, s);
-    else if (pr == ASX_C2P_ENTROPY) c2p_main_t<false, ASX_C2P_ENTROPY>(P, b, eos, a, hist, queue, qcount, s);
-    else c2p_main_t<false, ASX_C2P_PALENZUELA>(P, b, eos, a, hist, queue, qcount, s);
-  }
+hipError_t launch_con2prim_one(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
+                               bool from_A, unsigned long long *hist, hipStream_t s) {
+  c2p_one_t(P, c2p_box(P), eos, a, from_A, hist, s);
   return hipGetLastError();
 }
+hipError_t launch_con2prim_one(const KPatch &P, const TabEOS &eos, const C2PArgs &a,
+                               bool from_A, unsigned long long *hist, hipStream_t s) {
+  c2p_one_t(P, c2p_box(P), eos, a, from_A, hist, s);
+  return hipGetLastError();
+}
+
 hipError_t launch_con2prim_main(const KPatch &P, const TabEOS &eos, const C2PArgs &a,
                                 bool from_A, unsigned long long *hist, int *queue,
                                 unsigned *qcount, hipStream_t s) {
   const Box b = c2p_box(P);
   hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, qcount);
-  if (b.htotal() <= 0) return hipGetLastError();
-  if (from_A) c2p_main_t<true, ASX_C2P_PALENZUELA>(P, b, eos, a, hist, queue, qcount, s);
-  else c2p_main_t<false, ASX_C2P_PALENZUELA>(P, b, eos, a, hist, queue, qcount, s);
-  return hipGetLastError();
-}
-
-hipError_t launch_con2prim_rest(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
-                                bool from_A, unsigned long long *hist, const int *queue,
-                                const unsigned *qcount, hipStream_t s) {
-  const Box b = c2p_box(P);
-  if (b.htotal() <= 0) return hipSuccess;
-  c2p_rest_t(P, b, eos, a, from_A, hist, queue, qcount, s);
+  if (from_A)
+    hipLaunchKernelGGL((k_c2p_main<true, TabEOS>), b.grid(), dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
+  else
+    hipLaunchKernelGGL((k_c2p_main<false, TabEOS>), b.grid(), dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
   return hipGetLastError();
 }
 hipError_t launch_con2prim_rest(const KPatch &P, const TabEOS &eos, const C2PArgs &a,
                                 bool from_A, unsigned long long *hist, const int *queue,
                                 const unsigned *qcount, hipStream_t s) {
   const Box b = c2p_box(P);
-  if (b.htotal() <= 0) return hipSuccess;
-  c2p_rest_t(P, b, eos, a, from_A, hist, queue, qcount, s);
-  return hipGetLastError();
-}
-
-hipError_t launch_con2prim_main_batch(const KPatch *tab, const int *zbase, int np,
-                                      const IdealGas &eos, const C2PArgs &a,
-                                      const BatchRef *map, int nmap, int *queue,
-                                      unsigned *qcount, hipStream_t s) {
-  (void)np;
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, qcount);
-  if (nmap <= 0) return hipGetLastError();
-  const dim3 grid((unsigned)nmap), block(256);
-  if (a.prime == ASX_C2P_NOBLE)
-    hipLaunchKernelGGL(k_c2p_main_batch<ASX_C2P_NOBLE>, grid, block, 0, s, tab, zbase, eos, a, map, nmap, queue, qcount);
-  else if (a.prime == ASX_C2P_ENTROPY)
-    hipLaunchKernelGGL(k_c2p_main_batch<ASX_C2P_ENTROPY>, grid, block, 0, s, tab, zbase, eos, a, map, nmap, queue, qcount);
+  // enough work-items for a few percent of the zones; more stride
+  const dim3 grid((unsigned)std::min<int64_t>((b.htotal() + 255) / 256, 2048));
+  if (from_A)
+    hipLaunchKernelGGL((k_c2p_rest<true, TabEOS>), grid, dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
   else
-    hipLaunchKernelGGL(k_c2p_main_batch<ASX_C2P_PALENZUELA>, grid, block, 0, s, tab, zbase, eos, a, map, nmap, queue, qcount);
+    hipLaunchKernelGGL((k_c2p_rest<false, TabEOS>), grid, dim3(256), 0, s, P, b, eos, a, hist, queue, qcount);
   return hipGetLastError();
 }
 
-hipError_t launch_con2prim_rest_batch(const KPatch *tab, const int *zbase, int np,
-                                      const IdealGas &eos, const C2PArgs &a, int64_t nzones,
-                                      const int *queue, const unsigned *qcount,
-                                      hipStream_t s) {
-  if (nzones <= 0 || np <= 0) return hipSuccess;
-  const unsigned g2 = (unsigned)((nzones + 255) / 256 < 2048 ? (nzones + 255) / 256 : 2048);
-  hipLaunchKernelGGL(k_c2p_rest_batch, dim3(g2), dim3(256), 0, s, tab, zbase, np, eos, a, queue, qcount);
+hipError_t launch_con2prim_patches(const KPatch *tab, const IdealGas &eos, const C2PArgs &a,
+                                   const BatchRef *map, int nmap, hipStream_t s) {
+  if (nmap <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_c2p_patches, dim3((unsigned)nmap), dim3(256), 0, s, tab, eos, a, map, nmap);
   return hipGetLastError();
 }
 
@@ -264,8 +286,21 @@ hipError_t launch_c2p_batch(int64_t nz, const double *cons, const double *g,
                             int32_t *iters, const IdealGas &eos, const C2PArgs &a,
                             hipStream_t s) {
   if (nz <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_c2p_batch, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, s, nz,
-                     cons, g, seed, prim, flag, iters, eos, a);
+  const dim3 grid((unsigned)((nz + 255) / 256)), block(256);
+  if (nz <= kOnePassZones) {
+    hipLaunchKernelGGL(k_c2p_batch, grid, block, 0, s, nz, cons, g, seed, prim, flag, iters, eos, a);
+    return hipGetLastError();
+  }
+  if (a.prime == ASX_C2P_NOBLE)
+    hipLaunchKernelGGL(k_c2p_zones<ASX_C2P_NOBLE>, grid, block, 0, s, nz, cons, g, seed, prim, flag, iters, eos, a);
+  else if (a.prime == ASX_C2P_ENTROPY)
+    hipLaunchKernelGGL(k_c2p_zones<ASX_C2P_ENTROPY>, grid, block, 0, s, nz, cons, g, seed, prim, flag, iters, eos, a);
+  else
+    hipLaunchKernelGGL(k_c2p_zones<ASX_C2P_PALENZUELA>, grid, block, 0, s, nz, cons, g, seed, prim, flag, iters, eos, a);
+  // one wavefront for each of the 1024 SIMDs
+  const int per = (int)std::min<int64_t>(kRestZones, (nz / 1024 + 64) / 64 * 64);
+  hipLaunchKernelGGL(k_c2p_zones_rest, dim3((unsigned)((nz + per - 1) / per)), dim3(64), 0, s,
+                     nz, per, cons, g, seed, prim, flag, iters, eos, a);
   return hipGetLastError();
 }
 

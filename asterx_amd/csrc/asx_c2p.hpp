@@ -49,7 +49,8 @@ struct Cons {
     dB[0] *= s; dB[1] *= s; dB[2] *= s;
     DYe *= s; DEnt *= s;
   }
-  ASX_DEV void divide(double s) {
+  ASX_DEV void divide(double by) {
+    const Divisor s(by);
     dens /= s; tau /= s;
     mom[0] /= s; mom[1] /= s; mom[2] /= s;
     dB[0] /= s; dB[1] /= s; dB[2] /= s;
@@ -306,28 +307,30 @@ ASX_DEV void vel_from_Z(double Z, double W, double Bsq, double BiSi, const Cons 
                         const Sym3 &gup, const Sym3 &glo, bool use_z, Prim &pv) {
   const double *m = cv.mom;
   const double *B = cv.dB;
+  const Divisor zb(Z + Bsq), zzb(Z * (Z + Bsq));
   if (use_z) {
-    double zx = W * (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / (Z + Bsq);
-    zx += W * BiSi * B[0] / (Z * (Z + Bsq));
-    double zy = W * (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / (Z + Bsq);
-    zy += W * BiSi * B[1] / (Z * (Z + Bsq));
-    double zz = W * (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / (Z + Bsq);
-    zz += W * BiSi * B[2] / (Z * (Z + Bsq));
+    double zx = W * (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / zb;
+    zx += W * BiSi * B[0] / zzb;
+    double zy = W * (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / zb;
+    zy += W * BiSi * B[1] / zzb;
+    double zz = W * (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / zb;
+    zz += W * BiSi * B[2] / zzb;
     const double zxd = glo.xx * zx + glo.xy * zy + glo.xz * zz;
     const double zyd = glo.xy * zx + glo.yy * zy + glo.yz * zz;
     const double zzd = glo.xz * zx + glo.yz * zy + glo.zz * zz;
     const double lor = sqrt(1.0 + (zx * zxd + zy * zyd + zz * zzd));
-    pv.vel[0] = zx / lor;
-    pv.vel[1] = zy / lor;
-    pv.vel[2] = zz / lor;
+    const Divisor dl(lor);
+    pv.vel[0] = zx / dl;
+    pv.vel[1] = zy / dl;
+    pv.vel[2] = zz / dl;
     pv.w_lor = lor;
   } else {
-    pv.vel[0] = (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / (Z + Bsq);
-    pv.vel[0] += BiSi * B[0] / (Z * (Z + Bsq));
-    pv.vel[1] = (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / (Z + Bsq);
-    pv.vel[1] += BiSi * B[1] / (Z * (Z + Bsq));
-    pv.vel[2] = (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / (Z + Bsq);
-    pv.vel[2] += BiSi * B[2] / (Z * (Z + Bsq));
+    pv.vel[0] = (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / zb;
+    pv.vel[0] += BiSi * B[0] / zzb;
+    pv.vel[1] = (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / zb;
+    pv.vel[1] += BiSi * B[1] / zzb;
+    pv.vel[2] = (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / zb;
+    pv.vel[2] += BiSi * B[2] / zzb;
     pv.w_lor = W;
   }
 }
@@ -410,17 +413,26 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
   else if (x1 >= 1.0) x1 = dv;
   if (x0 <= 0.0) x0 = fabs(x0) + Zmin;
   else if (x0 > 1e20) x0 = xo0;
-  double errx = 1., df = 1., f = 1.;
+  double dx0 = 1., df = 1., f = 1.;
+  bool conv = false;
+  // What a step costs is its divisions.  The residuals r0 and r1 keep the
+  // reference's roundings (1/Z and the quotient by Gamma are rounded
+  // quotients); the derivatives, whose rounding the next step corrects, take
+  // the factor (Gamma - 1)/Gamma and reciprocals good to about a unit in the
+  // last place, and the step is compared with tol |Z| instead of divided by
+  // Z: seven divisions a step become two reciprocals and an estimate.
+  const Divisor dG(G);
+  const double gfac = (G - 1.0) * dG.r;
   int k;
   for (k = 1; k <= a.max_iter; k++) {
     const double Z = x0;
-    const double invZ = 1.0 / Z;
+    const double invZ = rcp_normal(Z);
     const double Vsq = x1;
     const double Sdotn = -(cv.tau + cv.dens);
     const double sq1v = sqrt(1.0 - Vsq);
-    const double p_tmp = ((Z * (1.0 - Vsq) - cv.dens * sq1v) * (G - 1.0) / (G));
-    const double dPdvsq = ((-Z + cv.dens / (2.0 * sq1v)) * (G - 1.0) / G);
-    const double dPdZ = ((1.0 - Vsq) * (G - 1.0) / G);
+    const double p_tmp = (Z * (1.0 - Vsq) - cv.dens * sq1v) * (G - 1.0) / dG;
+    const double dPdvsq = (-Z + 0.5 * cv.dens * rcp_normal(sq1v)) * gfac;
+    const double dPdZ = (1.0 - Vsq) * gfac;
     const double j00 = -2 * (Vsq + BiSi * BiSi * invZ * invZ * invZ) * (Bsq + Z);
     const double j01 = -(Bsq + Z) * (Bsq + Z);
     const double j10 = -1.0 + dPdZ - BiSi * BiSi * invZ * invZ * invZ;
@@ -432,8 +444,8 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
     const double detjac =
         (Bsq + Z) * (j10 * (Bsq + Z) +
                      (Bsq - 2.0 * dPdvsq) * (BiSi * BiSi * invZ * invZ + Vsq * Z) * invZ);
-    const double detjac_inv = 1.0 / detjac;
-    const double dx0 = -(j11 * r0 - j01 * r1) * detjac_inv;
+    const double detjac_inv = rcp_normal(detjac);
+    dx0 = -(j11 * r0 - j01 * r1) * detjac_inv;
     const double dx1 = -(-j10 * r0 + j00 * r1) * detjac_inv;
     df = -r0 * r0 - r1 * r1;
     f = -0.5 * (df);
@@ -444,11 +456,12 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
     else if (x1 >= 1.0) x1 = dv;
     if (x0 <= 0.0) x0 = fabs(x0) + Zmin;
     else if (x0 > 1e20) x0 = xo0;
-    errx = (x0 == 0.) ? fabs(dx0) : fabs(dx0 / x0);
-    if (fabs(errx) <= a.tol) break;
+    conv = fabs(dx0) <= (x0 == 0. ? a.tol : a.tol * fabs(x0));
+    if (conv) break;
   }
   rep.iters = k;
-  if (fabs(errx) > a.tol) {
+  const double errx = (x0 == 0.) ? fabs(dx0) : fabs(dx0 / x0);
+  if (!conv && errx > a.tol) {
     rep.status = ST_ROOT_FAIL_CONV; rep.adjust_cons = true;
     cv.scale(sqrt_detg);
     return;
@@ -866,7 +879,8 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
   const double sqrt_detg = sqrt(det3(glo));
   Cons cv = in.cv;
   double Bup[3];
-  for (int i = 0; i < 3; ++i) Bup[i] = cv.dB[i] / sqrt_detg;
+  const Divisor ds(sqrt_detg);
+  for (int i = 0; i < 3; ++i) Bup[i] = cv.dB[i] / ds;
   Prim pv;
   prim_nan(pv);
   Prim seed;

@@ -1075,30 +1075,37 @@ static asx_status c2p_common(const asx_patch *pt, const asx_params *par, bool fr
     }
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, s, cd, 80);
   }
-  int *queue;
-  unsigned *qcount;
-  if (fixed) {
-    queue = fixed->queue;
-    qcount = fixed->qcount;
-  } else {
-    C2PQueue *Q = c2p_queue(stream, (int64_t)pt->n[0] * pt->n[1] * pt->n[2]);
-    if (!Q) return ASX_ERR_DEVICE;
-    queue = Q->q;
-    qcount = Q->n;
-  }
+  const int64_t nz = (int64_t)pt->n[0] * pt->n[1] * pt->n[2];
   const C2PArgs ca = c2p_args(par);
   unsigned long long *hist = cd ? cd + 2 : nullptr;
   const bool tab = tabulated(par);
-  if ((st = dev_status(run(ASX_KC_C2P, [&] {
-         return tab ? launch_con2prim_main(P, tab_eos(par), ca, from_A, hist, queue, qcount, s)
-                    : launch_con2prim_main(P, ideal_gas(par), ca, from_A, hist, queue, qcount, s);
-       }))))
-    return st;
-  if ((st = dev_status(run(ASX_KC_C2P_REST, [&] {
-         return tab ? launch_con2prim_rest(P, tab_eos(par), ca, from_A, hist, queue, qcount, s)
-                    : launch_con2prim_rest(P, ideal_gas(par), ca, from_A, hist, queue, qcount, s);
-       }))))
-    return st;
+  if (!tab || nz <= kOnePassTableZones) {
+    if ((st = dev_status(run(ASX_KC_C2P, [&] {
+           return tab ? launch_con2prim_one(P, tab_eos(par), ca, from_A, hist, s)
+                      : launch_con2prim_one(P, ideal_gas(par), ca, from_A, hist, s);
+         }))))
+      return st;
+  } else {
+    int *queue;
+    unsigned *qcount;
+    if (fixed) {
+      queue = fixed->queue;
+      qcount = fixed->qcount;
+    } else {
+      C2PQueue *Q = c2p_queue(stream, nz);
+      if (!Q) return ASX_ERR_DEVICE;
+      queue = Q->q;
+      qcount = Q->n;
+    }
+    if ((st = dev_status(run(ASX_KC_C2P, [&] {
+           return launch_con2prim_main(P, tab_eos(par), ca, from_A, hist, queue, qcount, s);
+         }))))
+      return st;
+    if ((st = dev_status(run(ASX_KC_C2P_REST, [&] {
+           return launch_con2prim_rest(P, tab_eos(par), ca, from_A, hist, queue, qcount, s);
+         }))))
+      return st;
+  }
   if (cnt) {
     unsigned long long h[71];
     if (hipMemcpyAsync(h, cd + 2, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -2295,13 +2302,7 @@ asx_status plan_stage(asx_batch *b, int s, hipStream_t str) {
   const IdealGas eos = ideal_gas(&b->par);
   const C2PArgs ca = c2p_args(&b->par);
   if ((st = dev_status(timed(ASX_KC_C2P, str, [&] {
-         return launch_con2prim_main_batch(U, b->zbase, b->np, eos, ca, L->map, L->nmap,
-                                           b->queue, b->qcount, str);
-       }))))
-    return st;
-  if ((st = dev_status(timed(ASX_KC_C2P_REST, str, [&] {
-         return launch_con2prim_rest_batch(U, b->zbase, b->np, eos, ca, b->nzones, b->queue,
-                                           b->qcount, str);
+         return launch_con2prim_patches(U, eos, ca, L->map, L->nmap, str);
        }))))
     return st;
   return plan_bc(b, U, kSyncPrims, kNumSyncPrims, str);

@@ -316,16 +316,23 @@ hipError_t launch_update(const KPatch &P, const RhsArgs &A, const StatePtrs &u0,
                          const StatePtrs &out, double c0, double c1, double c2,
                          int variant, hipStream_t s);
 
+// con2prim of the patch interior in one pass over the full chain
+hipError_t launch_con2prim_one(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
+                               bool from_A, unsigned long long *hist, hipStream_t s);
+hipError_t launch_con2prim_one(const KPatch &P, const TabEOS &eos, const C2PArgs &a,
+                               bool from_A, unsigned long long *hist, hipStream_t s);
+// Independent zones, whose failures are scattered, take one pass while all
+// wavefronts are resident at the full chain's two per SIMD (2 x 4 x 256 of
+// 64): its registers then cost nothing, and the second pass is saved.
+constexpr int64_t kOnePassZones = 128 * 1024;
+// A patch on a table takes the two passes below beyond this many zones: the
+// table's full chain is the slower body (128^3, no failed zones: substep 2.33
+// ms in one pass, 2.15 in two), until the second pass costs as much (90^3
+// 0.82 / 0.86, after some substeps 0.69 / 0.89; 64^3 0.26 / 0.35).
+constexpr int64_t kOnePassTableZones = 1024 * 1024;
 // con2prim of the patch interior in two passes: every zone through the
 // primary solver, the zones it failed queued (queue: one int per interior
 // zone, qcount: one unsigned) and run through the full chain.
-hipError_t launch_con2prim_main(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
-                                bool from_A, unsigned long long *hist, int *queue,
-                                unsigned *qcount, hipStream_t s);
-hipError_t launch_con2prim_rest(const KPatch &P, const IdealGas &eos, const C2PArgs &a,
-                                bool from_A, unsigned long long *hist, const int *queue,
-                                const unsigned *qcount, hipStream_t s);
-// with a table: Palenzuela primary
 hipError_t launch_con2prim_main(const KPatch &P, const TabEOS &eos, const C2PArgs &a,
                                 bool from_A, unsigned long long *hist, int *queue,
                                 unsigned *qcount, hipStream_t s);
@@ -362,16 +369,9 @@ hipError_t launch_update_batch(const KPatch *tab, const StatePtrs *u0, const Sta
 // ghost layers normal to d, sized for the widest centering
 hipError_t launch_bc_batch(const KPatch *tab, const BCSlots &L, const BatchRef *map, int nmap,
                            int kind, hipStream_t s);
-// con2prim of the patch interiors; zbase[p] = first global zone of patch p
-// (np + 1 entries), the queue holds global zone indices
-hipError_t launch_con2prim_main_batch(const KPatch *tab, const int *zbase, int np,
-                                      const IdealGas &eos, const C2PArgs &a,
-                                      const BatchRef *map, int nmap, int *queue,
-                                      unsigned *qcount, hipStream_t s);
-hipError_t launch_con2prim_rest_batch(const KPatch *tab, const int *zbase, int np,
-                                      const IdealGas &eos, const C2PArgs &a, int64_t nzones,
-                                      const int *queue, const unsigned *qcount,
-                                      hipStream_t s);
+// con2prim of the patch interiors
+hipError_t launch_con2prim_patches(const KPatch *tab, const IdealGas &eos, const C2PArgs &a,
+                                   const BatchRef *map, int nmap, hipStream_t s);
 // A whole SSPRK3 stage of a batch as one persistent cooperative launch
 // (asx_plan.hip): the launch lists of each phase and everything the phases
 // read, in device memory.  Faces use tile variant 0 of every direction, the

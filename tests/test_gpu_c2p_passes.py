@@ -1,0 +1,131 @@
+"""Con2prim in one pass (few zones) and in two, a primary-only pass and the
+zones it failed, give the same bits."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from asterx_amd import abi
+from states import make_state, rel_err
+
+pytestmark = pytest.mark.gpu
+
+ONE_PASS = 128 * 1024  # zones, kOnePassZones
+
+
+def _torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+def _lib():
+    from asterx_amd import lib
+    return lib.lib()
+
+
+def _solve(par, cons, g, seed):
+    torch = _torch()
+    nz = cons.shape[1]
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (cons, g, seed)]
+    prim = torch.full((8, nz), -7.0, dtype=torch.float64, device="cuda")
+    flag = torch.full((nz,), -7.0, dtype=torch.float64, device="cuda")
+    it = torch.full((nz,), -7, dtype=torch.int32, device="cuda")
+    abi.check("asx_c2p_batch", _lib().asx_c2p_batch(
+        nz, t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), prim.data_ptr(),
+        flag.data_ptr(), it.data_ptr(), C.byref(par), None))
+    torch.cuda.synchronize()
+    return prim.cpu().numpy(), flag.cpu().numpy(), it.cpu().numpy()
+
+
+@pytest.mark.parametrize("prime,second", [("Noble", "Palenzuela"), ("Palenzuela", "Noble")])
+@pytest.mark.parametrize("nz", [ONE_PASS, ONE_PASS + 1, ONE_PASS + 4160])
+def test_zones(prime, second, nz):
+    from asterx_amd.zones import make_batch
+    n0 = 20011
+    cons, g, seed, _ = make_batch(n0, seed=5)
+    rng = np.random.default_rng(6)
+    bad = rng.random(n0) < 0.05  # seeds that make the primary fail, bad states
+    seed[:2, bad] *= 1e6
+    cons[4, ::997] = np.nan
+    cons[0, 1::1999] = 1e-14
+    cons[4, 2::1501] = np.inf
+    par = abi.params(gl_gamma=5.0 / 3.0, eps_max=1e8, rho_max=1e8, rho_abs_min=1e-12,
+                     vw_lim=1e3, B_lim=1e3, c2p_prime=prime, c2p_second=second)
+    one = _solve(par, cons, g, seed)
+    reps = -(-nz // n0)
+    two = _solve(par, *(np.tile(a, (1, reps))[:, :nz] for a in (cons, g, seed)))
+    # primary and atmosphere, and where Noble fails some the backup too
+    assert len(set(one[1])) > (2 if prime == "Noble" else 1)
+    for a, b in zip(one, two):
+        want = np.tile(a, reps)[..., :nz] if a.ndim == 1 else np.tile(a, (1, reps))[:, :nz]
+        assert np.array_equal(b, want, equal_nan=True)
+    assert (two[1] >= 0).all()
+
+
+@pytest.mark.parametrize("n", [(13, 12, 11), (70, 41, 50)])
+def test_patch_with_failures(n):
+    """A patch in which the primary fails here and there, against the oracle."""
+    torch = _torch()
+    h = make_state(n=n, curved=True)
+    dens, tau = h["dens"], h["tau"]
+    dens[5, 6, 7] = 1e-14
+    tau[7::5, 5, 6::7] *= 1e-6
+    tau[8, 5, 6] = np.nan
+    d = h.to("cuda")
+    par = abi.params(c2p_prime="Noble", c2p_second="Palenzuela", gl_gamma=5.0 / 3.0,
+                     rho_abs_min=1e-12)
+    cnt = abi.asx_counters()
+    abi.check("asx_con2prim", _lib().asx_con2prim(C.byref(d.struct()), C.byref(par),
+                                                  C.byref(cnt), None))
+    torch.cuda.synchronize()
+    abi.check("orc_con2prim", oracle.lib().orc_con2prim(C.byref(h.struct()), C.byref(par)))
+    sl = h.interior("rho")
+    fl = h.numpy("con2prim_flag")[sl]
+    assert np.array_equal(fl, d.numpy("con2prim_flag")[sl])
+    assert list(np.bincount(fl.astype(int).ravel(), minlength=7)) == list(cnt.c2p_flags)
+    assert len(np.unique(fl)) >= 3
+    for name in ("rho", "eps", "press", "velx", "Bvecz", "dens", "tau", "DEnt", "svec_y"):
+        assert rel_err(d.numpy(name)[sl], h.numpy(name)[sl]) <= 1e-9, name
+
+
+def test_table_patch():
+    """Past the table's line (1024^2 zones) the two passes, before it one: a
+    patch tiled from a small one, zone by zone the same bits."""
+    torch = _torch()
+    from asterx_amd import lib, tabeos
+    from asterx_amd.patch import Patch
+    table = tabeos.build()
+    kw = dict(c2p_prime="Palenzuela", c2p_second="None", use_temperature=1, use_press_atmo=0,
+              thermal_eos_atmo=1, t_atmo=0.01, Ye_atmo=0.3, c2p_tol=1e-10, max_iter=100,
+              vw_lim=1e3, B_lim=1e3, ye_min=0.035, ye_max=0.55, rho_abs_min=1e-12)
+    htab, dtab = tabeos.Table(table, device=None), tabeos.Table(table, device="cuda")
+    n0, n = (16, 16, 15), (128, 128, 66)
+    par = dtab.attach(abi.params(**kw))
+    src = make_state(n=n0, curved=False, table_par=htab.attach(abi.params(**kw)))
+    src["dens"][5, 6, 7] = 1e-25  # atmosphere
+    src["tau"][4::4, 5::5, 6::3] = -1.0  # floored
+    src["dens"][9, 9, 9] = np.nan
+    cells = abi.CONS + abi.DB + abi.SAVED + ["temperature"]
+    outs = abi.PRIMS + abi.CONS + abi.DB + abi.SAVED + abi.ZS + ["con2prim_flag"]
+    got = []
+    for m in (n0, n):
+        d = Patch(m, 3, src.x0, src.dx, slots=set(abi.ADM + cells + outs), device="cuda")
+        for name in ("alp", "gxx", "gyy", "gzz"):
+            d[name] = 1.0
+        for name in cells:
+            a = src.numpy(name)[src.interior(name)]
+            a = np.tile(a, [-(-m[2 - q] // n0[2 - q]) for q in range(3)])
+            full = np.zeros(d.shape(name))
+            full[d.interior(name)] = a[:m[2], :m[1], :m[0]]
+            d[name] = full
+        abi.check("asx_con2prim", lib.lib().asx_con2prim(C.byref(d.struct()), C.byref(par),
+                                                         None, None))
+        torch.cuda.synchronize()
+        got.append({k: d.numpy(k)[d.interior(k)] for k in outs})
+    assert len(np.unique(got[0]["con2prim_flag"])) >= 2
+    for k in outs:
+        a = np.tile(got[0][k], [-(-n[2 - q] // n0[2 - q]) for q in range(3)])
+        assert np.array_equal(got[1][k], a[:n[2], :n[1], :n[0]], equal_nan=True), k
