@@ -55,8 +55,10 @@ class Evolution:
         self.with_tmunu = tmunu
         self.fused = fused
 
-    def sync(self, names):
-        ps = self.p.struct()
+    # ps: the patch's struct, for callers that make several calls on it
+    def sync(self, names, ps=None):
+        if ps is None:
+            ps = self.p.struct()
         self.b.bc_fill_many(ps, [abi.SLOT[n] for n in names if n in self.p],
                             self.bc)
 
@@ -82,22 +84,24 @@ class Evolution:
             b.substep_bc(p.struct(), None, p.state(abi.STATE_RHS), 0.0, 0.0, 1.0, par,
                          self.bc)
             return
-        b.fluxes(p.struct(), par, 0)
-        self.sync(SYNC_FLUXES + (SYNC_UCT if self.uct else []))
-        b.source_terms(p.struct(), par)
-        self.sync(SYNC_RHS_HYDRO)
-        b.rhs(p.struct(), par)
-        self.sync(SYNC_RHS_HYDRO + SYNC_RHS_EM)
+        ps = p.struct()
+        b.fluxes(ps, par, 0)
+        self.sync(SYNC_FLUXES + (SYNC_UCT if self.uct else []), ps)
+        b.source_terms(ps, par)
+        self.sync(SYNC_RHS_HYDRO, ps)
+        b.rhs(ps, par)
+        self.sync(SYNC_RHS_HYDRO + SYNC_RHS_EM, ps)
 
     def poststep(self):
         p, b = self.p, self.b
-        self.sync(abi.STATE)
-        b.bstag_from_A(p.struct())
-        self.sync(abi.DBSTAG)
-        b.dB_from_bstag(p.struct())
-        self.sync(abi.DB)
-        b.con2prim(p.struct(), self.par)
-        self.sync(SYNC_C2P)
+        ps = p.struct()
+        self.sync(abi.STATE, ps)
+        b.bstag_from_A(ps)
+        self.sync(abi.DBSTAG, ps)
+        b.dB_from_bstag(ps)
+        self.sync(abi.DB, ps)
+        b.con2prim(ps, self.par)
+        self.sync(SYNC_C2P, ps)
         if self.with_tmunu:
             self.tmunu()
 
