@@ -10,8 +10,10 @@
 // LDS once per tile (coalesced rows, each cell fetched once), every
 // work-item reduces its (ORD x ORD) window of the plane in x and y from LDS,
 // and keeps the last ORD reduced planes of each variable in registers, so
-// the z reduction costs nothing extra.  The global loads of the next plane
-// are issued before the reductions of the current one.
+// the z reduction costs nothing extra.  EARLY: the global loads of the next
+// plane are issued before the reductions of the current one, else after its
+// results (order 4 of 193^3 vertices 0.84 -> 0.80 ms; order 2, whose planes
+// are fewer and reductions short, 0.65 ms late and 0.67 early).
 #include "asx_kernels.hpp"
 
 namespace asx {
@@ -129,9 +131,9 @@ template <int YS> ASX_DEV void tile_of(int b, int ntx, int nty, int ntz, int &bx
   }
 }
 
-template <int ORD, int TX, int TY, int TZ, int WAVES, int YS>
+template <int ORD, int TX, int TY, int WAVES, int YS, bool EARLY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_tmunu(
-    KPatch P, int ntx, int nty, int nb, int use_z) {
+    KPatch P, int ntx, int nty, int nb, int tz, int use_z) {
   using T = TmTile<ORD, TX, TY>;
   constexpr int H = T::H, CX = T::CX, NC = T::NC, PER = T::PER;
   __shared__ double lds[kTmunuVars][NC];
@@ -141,8 +143,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
   const int tid = (int)threadIdx.x, tx = tid % TX, ty = tid / TX;
   const int i0 = P.ng + bx * TX, j0 = P.ng + by * TY;
   const int i = i0 + tx, j = j0 + ty;
-  const int kb = P.ng + bz * TZ;
-  const int ke = min(kb + TZ, P.ng + P.n[2] + 1);
+  const int kb = P.ng + bz * tz;
+  const int ke = min(kb + tz, P.ng + P.n[2] + 1);
   const bool mine = i <= P.ng + P.n[0] && j <= P.ng + P.n[1];
   // last cell any interior vertex's stencil reads, per axis
   const int cxmax = P.ng + P.n[0] + H - 1, cymax = P.ng + P.n[1] + H - 1;
@@ -196,6 +198,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
       for (int r = 0; r < PER; ++r)
         if (tid + 256 * r < NC) lds[q][tid + 256 * r] = nxt[q][r];
     __syncthreads();
+    if (EARLY && p + 1 < np) fetch(kb - H + p + 1);
     double v[kTmunuVars];
 #pragma unroll
     for (int q = 0; q < kTmunuVars; ++q) {
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
       asm volatile("" : "+v"(ob));
       tmunu_point(P, use_z != 0, ob, v);
     }
-    if (p + 1 < np) fetch(kb - H + p + 1);
+    if (!EARLY && p + 1 < np) fetch(kb - H + p + 1);
   }
 }
 
@@ -233,19 +236,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
 // i-ORD/2 .. i+ORD/2-1 per axis, inside the patch for vertices ng..ng+n when
 // ng >= ORD/2 (checked by the caller); cells past the last one any interior
 // vertex needs are not read.
-template <int ORD, int TX, int TY, int TZ, int WAVES, int YS = 0>
+template <int ORD, int TX, int TY, int TZ, int WAVES, int YS = 0, bool EARLY = false>
 static hipError_t tmunu_t(const KPatch &P, int use_z, hipStream_t s) {
   const int ntx = (P.n[0] + 1 + TX - 1) / TX, nty = (P.n[1] + 1 + TY - 1) / TY;
-  const int ntz = (P.n[2] + 1 + TZ - 1) / TZ;
+  // Shorter runs where full ones leave CUs without the two workgroups that
+  // hide each other's latencies: a run of tz vertices reads ORD - 1 planes
+  // more than tz, but a march of 19 planes is 19 latencies long.  Order 4:
+  // 20 x 18 x 25 120 -> 26 us, 40 x 60 x 50 133 -> 38, 96 x 80 x 101 166 -> 112.
+  int tz = TZ;
+  while (tz > 2 && ntx * nty * ((P.n[2] + tz) / tz) < 512) tz /= 2;
+  const int ntz = (P.n[2] + 1 + tz - 1) / tz;
   const int nb = ntx * nty * ntz;
-  hipLaunchKernelGGL((k_tmunu<ORD, TX, TY, TZ, WAVES, YS>), dim3(nb), dim3(256), 0, s, P, ntx,
-                     nty, nb, use_z);
+  hipLaunchKernelGGL((k_tmunu<ORD, TX, TY, WAVES, YS, EARLY>), dim3(nb), dim3(256), 0, s, P, ntx,
+                     nty, nb, tz, use_z);
   return hipGetLastError();
 }
 
 template <int ORD>
 static hipError_t tmunu_v(const KPatch &P, int use_z, int variant, hipStream_t s) {
-  // default: 32 x 8 columns at a 3-wave register budget (0.83-0.89 ms for
+  // default: 32 x 8 columns at a 3-wave register budget (0.80 ms for
   // order 4 on 193^3 vertices; the other shapes 0.93-0.98 ms; the banded
   // orders 7 and 8 measure within the same run-to-run spread)
   switch (variant) {
@@ -257,7 +266,7 @@ static hipError_t tmunu_v(const KPatch &P, int use_z, int variant, hipStream_t s
   case 6: return tmunu_t<ORD, 64, 4, 16, 3>(P, use_z, s);
   case 7: return tmunu_t<ORD, 32, 8, 16, 3, 2>(P, use_z, s);
   case 8: return tmunu_t<ORD, 32, 8, 16, 3, 4>(P, use_z, s);
-  default: return tmunu_t<ORD, 32, 8, 16, 3>(P, use_z, s);
+  default: return tmunu_t<ORD, 32, 8, 16, 3, 0, ORD == 4>(P, use_z, s);
   }
 }
 

@@ -84,3 +84,66 @@ def test_faces_in_one_launch(n, recon, halo):
             abi.check("asx_set_variant", L.asx_set_variant(kc, 0))
     for m in names:
         assert np.array_equal(got[0][m], got[1][m]), m
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("n,nz", [((160, 90, 130), 9), ((40, 20, 60), 1), ((5, 3, 17), 4)])
+def test_tmunu_runs(order, n, nz):
+    """The tensor does not depend on the length of the runs along z, which the
+    number of tiles sets: a patch against a slab of it."""
+    torch = _torch()
+    L, ng = _lib(), 2
+    par = abi.params(tmunu_interp_order=order)
+    fields = abi.PRIMS + abi.ADM[:10]
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    p = Patch(n, ng, (0, 0, 0), (1, 1, 1), slots=fields + abi.TMUNU, device="cuda")
+    z0 = n[2] // 3
+    q = Patch((n[0], n[1], nz), ng, (0, 0, 0), (1, 1, 1), slots=fields + abi.TMUNU,
+              device="cuda")
+    for name in fields:
+        p[name].copy_(torch.rand(p.shape(name), dtype=torch.float64, device="cuda",
+                                 generator=gen) * 0.1)
+        if name in ("alp", "gxx", "gyy", "gzz"):
+            p[name].add_(1.0)
+        q[name].copy_(p[name][z0:z0 + q.shape(name)[0]])
+    for d in (p, q):
+        abi.check("asx_tmunu", L.asx_tmunu(C.byref(d.struct()), C.byref(par), None))
+    torch.cuda.synchronize()
+    for name in abi.TMUNU:
+        a = p[name][ng + z0:ng + z0 + nz + 1, ng:ng + n[1] + 1, ng:ng + n[0] + 1]
+        assert torch.equal(a, q[name][q.interior(name)]), name
+        assert bool((a != 0).all())
+    p["eTtt"][p.interior("eTtt")].zero_()
+    assert bool((p["eTtt"] == 0).all())  # nothing outside the interior
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("n", [(15, 15, 15), (16, 17, 18), (63, 31, 30), (64, 31, 31)])
+def test_update_with_every_load_in_flight(n, order):
+    """The small-patch update (16 x 2 x 2 tiles up to 1024 of them) against the
+    tiled one, on either side of that line."""
+    torch = _torch()
+    from asterx_amd.patch import StateBuf
+    L, kc = _lib(), abi.KCLASS["update"]
+    par = abi.params(reconstruction_method="wenoz", flux_type="HLLE", local_spatial_order=order)
+    d = make_state(n=n, curved=True).to("cuda")
+    u0 = StateBuf(d)
+    for name in abi.STATE:
+        u0.arr[name] = d[name].clone() * 1.01
+    got = []
+    try:
+        for v in (0, 1):
+            abi.check("asx_set_variant", L.asx_set_variant(kc, v))
+            out = StateBuf(d, fill=0.0)
+            abi.check("asx_substep", L.asx_substep(
+                C.byref(d.struct()), C.byref(u0.struct()), C.byref(out.struct()), 0.75, 0.25,
+                0.0025, C.byref(par), None))
+            torch.cuda.synchronize()
+            got.append({m: out.arr[m].cpu().numpy() for m in abi.STATE})
+    finally:
+        abi.check("asx_set_variant", L.asx_set_variant(kc, 0))
+    for m in abi.STATE:
+        # the sums contract multiply-adds as each kernel is compiled: a right-hand
+        # side of some 40 terms, 1.1e-16 each, times c2 = 0.0025
+        scale = np.abs(got[1][m]).max()
+        assert np.abs(got[0][m] - got[1][m]).max() <= 1e-14 * scale, m
