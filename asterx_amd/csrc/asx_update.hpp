@@ -67,16 +67,21 @@ ASX_DEV double corner_d2(const double c[8], int d, double idx) {
 // next field are not hoisted above the arithmetic of the previous one.  It
 // bounds how many stencil loads a work-item keeps in flight (each in-flight
 // double holds two VGPRs) and with it the register footprint.
-ASX_DEV void load_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
+// WIDE: no fence, every field's loads in flight together -- for patches so
+// small that each wavefront has a SIMD and its registers to itself, where the
+// fields' latencies one after another are what an update takes.
+template <bool WIDE> ASX_DEV void load_fence() {
+  if constexpr (!WIDE) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // Gradient of vertex field g at cell (vertex base o), order 2 or 4.
-template <int ORD>
+template <int ORD, bool WIDE>
 ASX_DEV void cell_grad(const KPatch &P, const double *g, int o, double out[3]) {
   const int sj = P.sj[7], sk = P.sk[7];
-  load_fence();
+  load_fence<WIDE>();
   if (ORD == 2) {
     double c[8];
     corners(g, o, sj, sk, c);
@@ -88,8 +93,8 @@ ASX_DEV void cell_grad(const KPatch &P, const double *g, int o, double out[3]) {
   }
 }
 // Cell average of vertex field g, fenced like cell_grad.
-ASX_DEV double cell_avg(const double *g, int o, int sj, int sk) {
-  load_fence();
+template <bool WIDE> ASX_DEV double cell_avg(const double *g, int o, int sj, int sk) {
+  load_fence<WIDE>();
   return avg_v2c(g, o, sj, sk);
 }
 
@@ -102,7 +107,7 @@ ASX_DEV double cell_avg(const double *g, int o, int sj, int sk) {
 //   C_ab = w_ab (T^00 beta^a beta^b + T^ab) / 2 + (t0^a beta^b + t0^b beta^a) / (1 + [a==b]),
 // (w_ab = 1 on, 2 off the diagonal), which is source.cxx:138-150 regrouped
 // by derivative, so that each derivative is consumed as it is loaded.
-template <int ORD>
+template <int ORD, bool WIDE = false>
 ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
                          double r[7]) {
   ASX_CONTRACT
@@ -119,12 +124,12 @@ ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
 #pragma unroll
     for (int d = 0; d < 3; ++d) d_alp[d] = fdv(d, P.g[ASX_ALP], ov, sj, sk, 4, P.idx[d]);
   }
-  const double beta[3] = {cell_avg(P.g[ASX_BETAX], ov, sj, sk),
-                          cell_avg(P.g[ASX_BETAY], ov, sj, sk),
-                          cell_avg(P.g[ASX_BETAZ], ov, sj, sk)};
-  const Sym3 g{cell_avg(P.g[ASX_GXX], ov, sj, sk), cell_avg(P.g[ASX_GXY], ov, sj, sk),
-               cell_avg(P.g[ASX_GXZ], ov, sj, sk), cell_avg(P.g[ASX_GYY], ov, sj, sk),
-               cell_avg(P.g[ASX_GYZ], ov, sj, sk), cell_avg(P.g[ASX_GZZ], ov, sj, sk)};
+  const double beta[3] = {cell_avg<WIDE>(P.g[ASX_BETAX], ov, sj, sk),
+                          cell_avg<WIDE>(P.g[ASX_BETAY], ov, sj, sk),
+                          cell_avg<WIDE>(P.g[ASX_BETAZ], ov, sj, sk)};
+  const Sym3 g{cell_avg<WIDE>(P.g[ASX_GXX], ov, sj, sk), cell_avg<WIDE>(P.g[ASX_GXY], ov, sj, sk),
+               cell_avg<WIDE>(P.g[ASX_GXZ], ov, sj, sk), cell_avg<WIDE>(P.g[ASX_GYY], ov, sj, sk),
+               cell_avg<WIDE>(P.g[ASX_GYZ], ov, sj, sk), cell_avg<WIDE>(P.g[ASX_GZZ], ov, sj, sk)};
   const double detg = det3(g);
   const double sqrt_detg = sqrt(detg);
   const Sym3 ug = inv3(g, detg);
@@ -191,12 +196,12 @@ ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
         dk[x == 0 ? y : (x == 1 ? 2 + y : 5)] =
             wab * (t00 * beta[x] * beta[y] + t(x, y)) + cross;
       }
-#pragma unroll 1
+#pragma unroll WIDE ? 6 : 1
     for (int f = 0; f < 6; ++f) {
       double c = dk[0];
 #pragma unroll
       for (int q = 1; q < 6; ++q) c = (f == q) ? dk[q] : c;
-      tau_source += c * cell_avg(P.g[ASX_KXX + f], ov, sj, sk);
+      tau_source += c * cell_avg<WIDE>(P.g[ASX_KXX + f], ov, sj, sk);
     }
   }
   double ms[3];
@@ -217,13 +222,13 @@ ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
       cf[3 + (x == 0 ? y : (x == 1 ? 2 + y : 5))] =
           0.5 * wab * (t00 * beta[x] * beta[y] + t(x, y)) + cross;
     }
-  // one field per iteration (not unrolled), so only that field's corner
-  // values are live
-#pragma unroll 1
+  // one field per iteration (not unrolled unless WIDE), so only that field's
+  // corner values are live
+#pragma unroll WIDE ? 9 : 1
   for (int f = 0; f < 9; ++f) {
     const int slot = f < 3 ? ASX_BETAX + f : ASX_GXX + (f - 3);
     double dq[3];
-    cell_grad<ORD>(P, P.g[slot], ov, dq);
+    cell_grad<ORD, WIDE>(P, P.g[slot], ov, dq);
     double c = cf[0];
 #pragma unroll
     for (int q = 1; q < 9; ++q) c = (f == q) ? cf[q] : c;
@@ -485,14 +490,14 @@ ASX_DEV constexpr int kSrcState(int q) {
 // waves per SIMD the register budget is sized for (order-4 derivatives
 // need 32 more doubles live than order 2)
 template <int ORD> constexpr int kUpdateWaves = ORD == 2 ? 4 : 3;
-template <int ORD>
+template <int ORD, bool WIDE = false>
 ASX_DEV void update_point(const KPatch &P, int i, int j, int k, const RhsArgs &A,
                           const StatePtrs &u0, const StatePtrs &out, const Comb &cb) {
   ASX_CONTRACT
   const bool cx = i < P.ng + P.n[0], cy = j < P.ng + P.n[1], cz = k < P.ng + P.n[2];
   if (cx && cy && cz) {
     double r[7];
-    source_cell<ORD>(P, i, j, k, A, r);
+    source_cell<ORD, WIDE>(P, i, j, k, A, r);
     const int oc = off(P, 0, i, j, k);
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
