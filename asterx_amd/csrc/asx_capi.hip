@@ -2075,13 +2075,15 @@ enum BatchKind {
   BK_BC = 5,     // ghost layers (bc_point's workgroups)
   BK_UBSTAG = 6, // + d: interior faces of the caller's dB_stag
   BK_C2P = 9,    // interior cells
-  BK_COUNT = 10
+  BK_COUNT = 10,
+  BK_FACES = 10 // faces of every direction and vertices (plan_faces)
 };
 
 struct BatchLaunch {
   BatchBox *box = nullptr;
   BatchRef *map = nullptr;
   int nmap = 0;
+  std::vector<BatchRef> refs; // map, on the host
 };
 
 } // namespace
@@ -2104,6 +2106,7 @@ struct asx_batch_s {
   int *queue = nullptr;
   unsigned *qcount = nullptr;
   std::map<std::pair<int, int>, BatchLaunch> launches; // (kind, variant)
+  KindBoxes fbox = {}; // of the list BK_FACES
   int var[4] = {0, 0, 0, 0}; // launch shapes: faces x, y, z, update
   hipStream_t cap = nullptr;
   hipGraph_t graph = nullptr;
@@ -2210,6 +2213,7 @@ asx_status plan_launch(asx_batch *b, int k, int v, BatchLaunch **out) {
   if (refs.size() >= (size_t(1) << 31)) return ASX_ERR_SIZE;
   BatchLaunch L;
   L.nmap = (int)refs.size();
+  L.refs = refs;
   asx_status st;
   if ((st = plan_upload(b, boxes, &L.box)) || (st = plan_upload(b, refs, &L.map))) return st;
   *out = &(b->launches[key] = L);
@@ -2240,13 +2244,61 @@ int plan_face_shape(const asx_batch *b, int d) {
   return b->var[d] ? b->var[d] : face_shape(d, b->par.reconstruction_method, false);
 }
 
+// The list of launch_faces_batch: each patch's tiles of the four kinds, patch
+// after patch.
+asx_status plan_faces(asx_batch *b, BatchLaunch **out) {
+  const auto key = std::make_pair((int)BK_FACES, 0);
+  auto it = b->launches.find(key);
+  if (it != b->launches.end()) {
+    *out = &it->second;
+    return ASX_OK;
+  }
+  BatchLaunch *K[4];
+  asx_status st;
+  for (int d = 0; d < 3; ++d)
+    if ((st = plan_launch(b, BK_FACE + d, face_shape(d, b->par.reconstruction_method, false), &K[d])))
+      return st;
+  if ((st = plan_launch(b, BK_AUX, 0, &K[3]))) return st;
+  int64_t n = 0;
+  for (int q = 0; q < 4; ++q) n += K[q]->nmap;
+  if (n >= (int64_t(1) << 31)) return ASX_ERR_SIZE;
+  std::vector<BatchRef> refs;
+  refs.reserve((size_t)n);
+  size_t at[4] = {0, 0, 0, 0};
+  for (int p = 0; p < b->np; ++p)
+    for (int q = 0; q < 4; ++q) {
+      const std::vector<BatchRef> &v = K[q]->refs;
+      for (; at[q] < v.size() && v[at[q]].pid == p; ++at[q])
+        refs.push_back(BatchRef{p | (q << kKindShift), v[at[q]].chunk});
+    }
+  for (int q = 0; q < 4; ++q) b->fbox.box[q] = K[q]->box;
+  BatchLaunch L;
+  L.nmap = (int)refs.size();
+  if ((st = plan_upload(b, refs, &L.map))) return st;
+  *out = &(b->launches[key] = L);
+  return ASX_OK;
+}
+// One launch, unless the caller has set or tuned a face shape or times the
+// kernel classes (a graph's launches are never timed).
+bool plan_one_launch(const asx_batch *b) {
+  return !(b->var[0] | b->var[1] | b->var[2]) && b->np < (1 << kKindShift) &&
+         (g_capturing || !g_timing.load(std::memory_order_relaxed));
+}
+
 asx_status plan_stencil(asx_batch *b, int s, hipStream_t str) {
   const int bi = kStageIn[s], bo = kStageOut[s];
   const KPatch *T = b->stab[bi];
   BatchLaunch *L;
   asx_status st;
   const FluxArgs A = plan_flux_args(&b->par);
-  for (int d = 0; d < 3; ++d) {
+  const bool one = plan_one_launch(b);
+  if (one) {
+    if ((st = plan_faces(b, &L))) return st;
+    if ((st = dev_status(launch_faces_batch(T, A, b->fbox, L->map, L->nmap,
+                                            b->par.reconstruction_method, str))))
+      return st;
+  }
+  for (int d = 0; d < 3 && !one; ++d) {
     const int v = plan_face_shape(b, d);
     if ((st = plan_launch(b, BK_FACE + d, v, &L))) return st;
     if ((st = dev_status(timed(ASX_KC_FACE_X + d, str, [&] {
@@ -2255,11 +2307,13 @@ asx_status plan_stencil(asx_batch *b, int s, hipStream_t str) {
          }))))
       return st;
   }
-  if ((st = plan_launch(b, BK_AUX, 0, &L))) return st;
-  if ((st = dev_status(timed(ASX_KC_AUX, str, [&] {
-         return launch_aux_batch(T, L->box, L->map, L->nmap, str);
-       }))))
-    return st;
+  if (!one) {
+    if ((st = plan_launch(b, BK_AUX, 0, &L))) return st;
+    if ((st = dev_status(timed(ASX_KC_AUX, str, [&] {
+           return launch_aux_batch(T, L->box, L->map, L->nmap, str);
+         }))))
+      return st;
+  }
   const int v = b->var[3];
   if ((st = plan_launch(b, BK_UPDATE, v, &L))) return st;
   const RhsArgs R = rhs_args(&b->par);
@@ -2319,7 +2373,7 @@ asx_status plan_prepare(asx_batch *b) {
     if (k == BK_UPDATE) v = b->var[3];
     if ((st = plan_launch(b, k, v, &L))) return st;
   }
-  return ASX_OK;
+  return plan_faces(b, &L);
 }
 
 void plan_drop_graph(asx_batch *b) {
@@ -2645,6 +2699,27 @@ asx_status asx_batch_autotune(asx_batch *plan, int32_t reps, void *stream) {
     }
   }
   for (int q = 0; q < 4; ++q) plan->var[q] = arg[q];
+  // the faces in one launch or one per direction in the shapes just found
+  if (!st && (arg[0] | arg[1] | arg[2]) && !(st = asx_timing_enable(0))) {
+    float ms[2] = {0, 0};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    if (hipEventCreate(&ev[0]) != hipSuccess || hipEventCreate(&ev[1]) != hipSuccess)
+      st = ASX_ERR_DEVICE;
+    for (int one = 0; one < 2 && !st; ++one) {
+      for (int q = 0; q < 3; ++q) plan->var[q] = one ? 0 : arg[q];
+      if ((st = plan_stencil(plan, 0, s))) break;
+      if (hipEventRecord(ev[0], s) != hipSuccess) st = ASX_ERR_DEVICE;
+      for (int r = 0; r < reps && !st; ++r) st = plan_stencil(plan, 0, s);
+      if (!st && (hipEventRecord(ev[1], s) != hipSuccess ||
+                  hipEventSynchronize(ev[1]) != hipSuccess ||
+                  hipEventElapsedTime(&ms[one], ev[0], ev[1]) != hipSuccess))
+        st = ASX_ERR_DEVICE;
+    }
+    if (st || ms[0] < ms[1])
+      for (int q = 0; q < 3; ++q) plan->var[q] = arg[q];
+    for (hipEvent_t x : ev)
+      if (x) (void)hipEventDestroy(x);
+  }
   {
     std::lock_guard<std::mutex> l(g_tmu);
     asx_status st2 = drain_timing();

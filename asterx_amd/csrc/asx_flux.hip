@@ -335,6 +335,33 @@ void k_face_batch(const KPatch *__restrict__ tab, FluxArgs A, const BatchBox *__
                      MB::ok ? MS : nullptr);
 }
 
+template <int M>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ASX_FACE_WAVES)))
+void k_faces_batch(const KPatch *__restrict__ tab, FluxArgs A, KindBoxes box,
+                   const BatchRef *__restrict__ map, int nmap) {
+  using T = FaceShapes<M, false>;
+  using MX = MetricBox<0, T::X>;
+  using MY = MetricBox<1, T::Y>;
+  using MZ = MetricBox<2, T::Z>;
+  constexpr int NX = MX::ok ? MX::N : 1, NY = MY::ok ? MY::N : 1, NZ = MZ::ok ? MZ::N : 1;
+  __shared__ FaceLDS S;
+  __shared__ double MS[NX > NY ? (NX > NZ ? NX : NZ) : (NY > NZ ? NY : NZ)];
+  const BatchRef r = map[xcd_tile((int)blockIdx.x, nmap)];
+  const int kind = r.pid >> kKindShift, pid = r.pid & ((1 << kKindShift) - 1);
+  const KPatch &P = tab[pid];
+  const BatchBox &bb = box.box[kind][pid];
+  if (kind == 0) {
+    face_tile<0, M, T::X>(P, A, bb.lo, bb.cnt, r.chunk, bb.nt[0], bb.nt[1], S, MX::ok ? MS : nullptr);
+  } else if (kind == 1) {
+    face_tile<1, M, T::Y>(P, A, bb.lo, bb.cnt, r.chunk, bb.nt[0], bb.nt[1], S, MY::ok ? MS : nullptr);
+  } else if (kind == 2) {
+    face_tile<2, M, T::Z>(P, A, bb.lo, bb.cnt, r.chunk, bb.nt[0], bb.nt[1], S, MZ::ok ? MS : nullptr);
+  } else {
+    int i, j, k;
+    if (batch_point(bb, r.chunk, i, j, k)) aux_point(P, i, j, k);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_aux_batch(const KPatch *__restrict__ tab,
                                                    const BatchBox *__restrict__ box,
                                                    const BatchRef *__restrict__ map, int nmap) {
@@ -415,6 +442,20 @@ hipError_t launch_face_batch(int d, const KPatch *tab, const FluxArgs &A, const 
   if (d == 0) launch_face_batch_d<0>(tab, A, box, map, nmap, method, variant, s);
   else if (d == 1) launch_face_batch_d<1>(tab, A, box, map, nmap, method, variant, s);
   else launch_face_batch_d<2>(tab, A, box, map, nmap, method, variant, s);
+  return hipGetLastError();
+}
+hipError_t launch_faces_batch(const KPatch *tab, const FluxArgs &A, const KindBoxes &box,
+                              const BatchRef *map, int nmap, int method, hipStream_t s) {
+  if (nmap <= 0) return hipSuccess;
+  const dim3 grid((unsigned)nmap), block(256);
+  switch (method) {
+  case ASX_RECON_GODUNOV: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_GODUNOV>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  case ASX_RECON_MINMOD: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_MINMOD>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  case ASX_RECON_MONOCENTRAL: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_MONOCENTRAL>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  case ASX_RECON_PPM: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_PPM>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  case ASX_RECON_WENOZ: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_WENOZ>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  default: hipLaunchKernelGGL(k_faces_batch<ASX_RECON_MP5>, grid, block, 0, s, tab, A, box, map, nmap); break;
+  }
   return hipGetLastError();
 }
 hipError_t launch_aux_batch(const KPatch *tab, const BatchBox *box, const BatchRef *map,

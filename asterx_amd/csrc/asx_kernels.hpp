@@ -356,6 +356,16 @@ struct BCSlots {
 hipError_t launch_face_batch(int d, const KPatch *tab, const FluxArgs &A, const BatchBox *box,
                              const BatchRef *map, int nmap, int method, int variant,
                              hipStream_t s);
+// The faces of every direction and the vertex auxiliaries in one launch, in
+// the shapes of face_shape(): map holds each patch's tiles of the four kinds
+// one after another, the kind (0..2 faces, 3 auxiliaries) in BatchRef::pid's
+// bits from kKindShift up; box[q]: the boxes of kind q.
+constexpr int kKindShift = 29;
+struct KindBoxes {
+  const BatchBox *box[4];
+};
+hipError_t launch_faces_batch(const KPatch *tab, const FluxArgs &A, const KindBoxes &box,
+                              const BatchRef *map, int nmap, int method, hipStream_t s);
 hipError_t launch_aux_batch(const KPatch *tab, const BatchBox *box, const BatchRef *map,
                             int nmap, hipStream_t s);
 // face B from the vector potential into each patch's dB_stag slot d
