@@ -946,9 +946,15 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
       palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, in.temperature, zguess, vguess, PRIME >= 0);
     }
     out.iters = rep1.iters;
-    if (PRIME >= 0 && rep1.failed()) return false;
+    // On a table without a backup the chain ends here (no guess that a second
+    // solve would do without): the zone need not repeat a primary of up to
+    // max_iter temperature solves to find that out.
+    constexpr bool ends = !std::is_same<E, IdealGas>::value;
+    if (PRIME >= 0 && rep1.failed() &&
+        !(ends && zguess < 0.0 && a.second != ASX_C2P_PALENZUELA))
+      return false;
+    if (rep1.failed()) code = ASX_C2P_FLAG_SECOND;
     if (PRIME < 0 && rep1.failed()) {
-      code = ASX_C2P_FLAG_SECOND;
       if constexpr (std::is_same<E, IdealGas>::value) {
         if (a.second == ASX_C2P_NOBLE) noble_solve(eos, atmo, a, pv, seed, cv, glo, rep2);
         else if (a.second == ASX_C2P_PALENZUELA) palenzuela_solve(eos, atmo, a, pv, cv, glo, rep2, in.temperature);
