@@ -453,7 +453,7 @@ enum { ASX_BC_LINEAR = 0, ASX_BC_PERIODIC = 1, ASX_BC_COPY = 2 };
 asx_status asx_bc_fill(const asx_patch *patch, int32_t slot, int32_t kind,
                        void *stream);
 /* The same fill for a list of grid functions (any centerings, at most 64) in
- * one launch per axis: the physical-boundary half of a SYNC statement with
+ * one launch: the physical-boundary half of a SYNC statement with
  * several groups (e.g. AsterX/schedule.ccl:78-81).  Same arguments and errors
  * as asx_bc_fill for each listed slot; ASX_ERR_PARAM for nslot > 64. */
 asx_status asx_bc_fill_many(const asx_patch *patch, int32_t nslot,
@@ -571,7 +571,8 @@ asx_status asx_release_scratch(void *stream);
  * reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops, harnesses that forbid hipMalloc).  The same
  * kernels and results as asx_con2prim_group; the queue of zones the primary
- * solver failed, its count and the counters live in a fixed device array
+ * solver failed (used with a table, beyond 1024^2 zones), its count and the
+ * counters live in a fixed device array
  * of the library (64 MiB + 2 KiB per device, held until the process ends)
  * instead of library-allocated buffers, and the launches are not timed
  * (asx_timing_*).  Patches of more than 2^24 interior zones: ASX_ERR_SIZE.
