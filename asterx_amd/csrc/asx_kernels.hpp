@@ -326,10 +326,10 @@ hipError_t launch_con2prim_one(const KPatch &P, const TabEOS &eos, const C2PArgs
 // 64): its registers then cost nothing, and the second pass is saved.
 constexpr int64_t kOnePassZones = 128 * 1024;
 // A patch on a table takes the two passes below beyond this many zones: the
-// table's full chain is the slower body (128^3, no failed zones: substep 2.33
-// ms in one pass, 2.15 in two), until the second pass costs as much (90^3
-// 0.82 / 0.86, after some substeps 0.69 / 0.89; 64^3 0.26 / 0.35).
-constexpr int64_t kOnePassTableZones = 1024 * 1024;
+// table's full chain is the slower body (128^3 substep 2.33 ms in one pass,
+// 2.15 in two; 90^3 0.85 / 0.79, 44^3 0.142 / 0.134, 64^3 0.256 / 0.266), and
+// below a wavefront per SIMD the launches saved weigh more.
+constexpr int64_t kOnePassTableZones = 64 * 1024;
 // con2prim of the patch interior in two passes: every zone through the
 // primary solver, the zones it failed queued (queue: one int per interior
 // zone, qcount: one unsigned) and run through the full chain.

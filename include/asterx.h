@@ -571,7 +571,7 @@ asx_status asx_release_scratch(void *stream);
  * reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops, harnesses that forbid hipMalloc).  The same
  * kernels and results as asx_con2prim_group; the queue of zones the primary
- * solver failed (used with a table, beyond 1024^2 zones), its count and the
+ * solver failed (used with a table, beyond 65536 zones), its count and the
  * counters live in a fixed device array
  * of the library (64 MiB + 2 KiB per device, held until the process ends)
  * instead of library-allocated buffers, and the launches are not timed

@@ -92,7 +92,7 @@ def test_patch_with_failures(n):
 
 
 def test_table_patch():
-    """Past the table's line (1024^2 zones) the two passes, before it one: a
+    """Past the table's line (65536 zones) the two passes, before it one: a
     patch tiled from a small one, zone by zone the same bits."""
     torch = _torch()
     from asterx_amd import lib, tabeos
@@ -102,7 +102,7 @@ def test_table_patch():
               thermal_eos_atmo=1, t_atmo=0.01, Ye_atmo=0.3, c2p_tol=1e-10, max_iter=100,
               vw_lim=1e3, B_lim=1e3, ye_min=0.035, ye_max=0.55, rho_abs_min=1e-12)
     htab, dtab = tabeos.Table(table, device=None), tabeos.Table(table, device="cuda")
-    n0, n = (16, 16, 15), (128, 128, 66)
+    n0, n = (16, 16, 15), (64, 33, 32)
     par = dtab.attach(abi.params(**kw))
     src = make_state(n=n0, curved=False, table_par=htab.attach(abi.params(**kw)))
     src["dens"][5, 6, 7] = 1e-25  # atmosphere
