@@ -152,7 +152,8 @@ class asx_eos_table(C.Structure):
                 ("nvars", C.c_int32), ("energy_shift", C.c_double),
                 ("eps_min", C.c_double), ("eps_max", C.c_double),
                 ("x_lo", C.c_double * 3), ("x_step", C.c_double * 3),
-                ("x_hi", C.c_double * 3)]
+                ("x_hi", C.c_double * 3), ("eps_grows_with_T", C.c_int32),
+                ("pad0", C.c_int32)]
 
 
 class asx_box(C.Structure):

@@ -270,6 +270,7 @@ TabEOS tab_eos(const asx_params *p) {
   e.ye_max = t->x_hi[2];
   e.eps_min = t->eps_min;
   e.eps_max = t->eps_max;
+  e.grows = t->eps_grows_with_T == 1;
   return e;
 }
 // An ideal gas or a table (entry points with composition)

@@ -119,6 +119,12 @@ int32_t asx_eos_read_stellarcollapse(const char *path, asx_eos_host_table *out) 
   // where the reference indexes its interleaved table as variable-major)
   out->eps_min = emin > 1e-15 ? emin : 1e-15;
   out->eps_max = emax;
+  const size_t line = 4 * (size_t)nrho, plane = line * ntemp;
+  bool grows = true;
+  for (size_t y = 0; y < (size_t)nye; ++y)
+    for (size_t q = y * plane + 1; q < (y + 1) * plane - line; q += 4) // log eps
+      grows = grows && out->data[q + line] - out->data[q] > 1e-12;
+  out->eps_grows_with_T = grows;
   return 0;
 }
 

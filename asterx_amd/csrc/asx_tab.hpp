@@ -23,6 +23,7 @@ struct TabEOS {
   double shift;         // energy shift
   double rho_min, rho_max, temp_min, temp_max, ye_min, ye_max; // rgrho, rgtemp, rgye
   double eps_min, eps_max;                                     // rgeps
+  int grows; // eps grows with T along every (rho, Ye) line (asx_eos_table)
 
   // nearest lower node, uniform axis (eos_linear_interp_ND.hxx:57-73)
   ASX_DEV int find(int d, double x) const {
@@ -109,18 +110,24 @@ struct TabEOS {
     return logtemp_nodes(lrho, leps, ye, vmin, vmax);
   }
   // The table cell of a zone's previous solve, kept in registers between the
-  // solves of one zone: node indices (i1 < 0: none yet), the cell's position
+  // solves of one zone: node indices (i0 < 0: none yet), the cell's position
   // and inverse width on each axis, and per corner [Ye][T][rho]
-  // log(eps + shift) and log p.
+  // log(eps + shift) and log p.  full: the next cell may not be looked for
+  // from this one, see solve_re.
   struct Cell {
     int i0 = -1, i1 = -1, i2 = 0;
+    bool full = false;
     double r0, ri, t0, dt, ly; // log rho: low node, 1 / width; log T: low node, width; Ye weight
     double e[2][2][2], p[2][2][2];
   };
   // Start of a zone's solves: its Ye, and a temperature near which to look.
+  // Between the Ye nodes a table that grows with T still grows; beyond them
+  // (by more than the rounding of the weight) the difference of two growing
+  // lines need not.
   ASX_DEV void start_cell(Cell &c, double ye, double temp) const {
     c.i2 = find(2, ye);
     c.ly = (ye - ax[2][c.i2]) / (ax[2][c.i2 + 1] - ax[2][c.i2]);
+    c.full = !(grows && c.ly >= -1e-15 && c.ly <= 1.0 + 1e-15);
     c.i1 = find(1, log(ctemp(temp)));
     c.i0 = -1;
   }
@@ -146,24 +153,27 @@ struct TabEOS {
           c.e[y][t][r] = v[EPS];
         }
   }
-  // p and log T from (rho, eps, Ye) with the zone's previous cell as the
-  // starting point: the same root as logtemp_re's for a table whose eps
-  // grows with T along each (rho, Ye) line (the bracketing cell is then
-  // unique), to rounding.  A zone's consecutive solves (the Brent iterates,
-  // then the final state) move rho and eps by less and less, so the cell
-  // they end in repeats: its corner values stay in registers and a solve
-  // inside it reads no memory.  When the root has left it, the next cell is
-  // predicted from the cell's slope d eps / d T (exact for a thermal energy
-  // linear in T, so it usually lands on the cell or beside it) and checked
-  // at its own nodes; a miss is searched outwards from there by doubling
-  // steps, then bisected.
+  // p and log T from (rho, eps, Ye): logtemp_re's root, to rounding.
+  // Where eps grows with T along the (rho, Ye) line one cell brackets the
+  // root, so the search may start anywhere, and starts from the zone's
+  // previous cell.  A zone's consecutive solves (the Brent
+  // iterates, then the final state) move rho and eps by less and less, so
+  // the cell they end in repeats: its corner values stay in registers and a
+  // solve inside it reads no memory.  When the root has left it, the next
+  // cell is predicted from the cell's slope d eps / d T (exact for a thermal
+  // energy linear in T, so it usually lands on the cell or beside it) and
+  // checked at its own nodes; a miss is searched outwards from there by
+  // doubling steps, then bisected.  Where eps need not grow (Cell::full)
+  // several cells may hold a root: the axis is bisected from its ends, as
+  // logtemp_re does it, and no result depends on where a search began.
   // Bound by the latency of dependent table reads: some lane of a wavefront
   // leaves its cell in almost every iteration, and a search from scratch
   // costs the whole wavefront eight dependent probes.  Con2prim of 1 000 003
   // zones on the 234 x 180 x 50 table: 2.75 ms with the search from scratch
   // outside the previous T cell, 0.79 ms with this (table reads per
-  // wavefront 1490 -> 436, waves waiting 74 % -> 34 % of their time);
-  // keeping the corners alone, without the prediction, left it at 2.70.
+  // wavefront 1490 -> 436, waves waiting 74 % -> 34 % of their time), 0.75
+  // since a predicted cell that holds is not loaded a second time; keeping
+  // the corners alone, without the prediction, left it at 2.70.
   ASX_DEV void solve_re(double rho, double &eps, Cell &c, double &lrho, double &lt,
                         double &press) const {
     const double r = crho(rho);
@@ -182,32 +192,39 @@ struct TabEOS {
     // outside [elo, ehi): every lane of the wavefront that has left its cell
     auto below = [&] { return !(elo <= leps); };
     auto above = [&] { return !(leps < ehi); };
-    if ((below() && c.i1 > 0) || (above() && c.i1 < last - 1)) {
-      // eps linear in T through the cell's nodes, in single precision
-      const float k = 1.44269504f;
-      const float dlo = __builtin_amdgcn_exp2f(k * (float)(elo - leps));
-      const float dhi = __builtin_amdgcn_exp2f(k * (float)(ehi - leps));
-      const float th = __builtin_amdgcn_exp2f(k * (float)c.dt);
-      // T / T_lo at the target
-      const float x = 1.0f + (1.0f - dlo) * (th - 1.0f) / (dhi - dlo);
-      const float step = __builtin_amdgcn_logf(fmaxf(x, 1e-30f)) / (k * (float)c.dt);
-      int j = c.i1 + (int)fminf(fmaxf(floorf(step), -(float)last), (float)last);
-      j = below() ? min(j, c.i1 - 1) : max(j, c.i1 + 1); // past the cell it left
-      j = min(max(j, 0), last - 1);
-      load_cell(c, i0, j);
-      elo = mix(c.e, 0);
-      ehi = mix(c.e, 1);
-      if ((below() && j > 0) || (above() && j < last - 1)) {
-        const int s1 = NV * n[0];
-        const double *row = tab + EPS + NV * i0 + s1 * n[1] * c.i2;
-        auto node = [&](int m) {
-          const double *q = row + s1 * m;
-          const int s2 = s1 * n[1];
-          const double a0 = (q[NV] - q[0]) * lr + q[0];
-          const double a1 = (q[s2 + NV] - q[s2]) * lr + q[s2];
-          return (a1 - a0) * c.ly + a0;
-        };
-        int lo = j, hi = j + 1, d = 1;
+    if (c.full || (below() && c.i1 > 0) || (above() && c.i1 < last - 1)) {
+      const int s1 = NV * n[0];
+      const double *row = tab + EPS + NV * i0 + s1 * n[1] * c.i2;
+      auto node = [&](int m) {
+        const double *q = row + s1 * m;
+        const int s2 = s1 * n[1];
+        const double a0 = (q[NV] - q[0]) * lr + q[0];
+        const double a1 = (q[s2 + NV] - q[s2]) * lr + q[s2];
+        return (a1 - a0) * c.ly + a0;
+      };
+      int lo, hi; // the root's cell is looked for between these nodes
+      if (c.full) {
+        const bool low = leps <= node(0), high = leps >= node(last);
+        lo = high && !low ? last - 1 : 0;
+        hi = low ? 1 : last;
+      } else {
+        // eps linear in T through the cell's nodes, in single precision
+        const float k = 1.44269504f;
+        const float dlo = __builtin_amdgcn_exp2f(k * (float)(elo - leps));
+        const float dhi = __builtin_amdgcn_exp2f(k * (float)(ehi - leps));
+        const float th = __builtin_amdgcn_exp2f(k * (float)c.dt);
+        // T / T_lo at the target
+        const float x = 1.0f + (1.0f - dlo) * (th - 1.0f) / (dhi - dlo);
+        const float step = __builtin_amdgcn_logf(fmaxf(x, 1e-30f)) / (k * (float)c.dt);
+        int j = c.i1 + (int)fminf(fmaxf(floorf(step), -(float)last), (float)last);
+        j = below() ? min(j, c.i1 - 1) : max(j, c.i1 + 1); // past the cell it left
+        j = min(max(j, 0), last - 1);
+        load_cell(c, i0, j);
+        elo = mix(c.e, 0);
+        ehi = mix(c.e, 1);
+        lo = j;
+        hi = j + 1;
+        int d = 1;
         if (below()) {
           while (lo > 0 && below()) {
             hi = lo;
@@ -223,15 +240,15 @@ struct TabEOS {
             ehi = node(hi);
           }
         }
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (node(mid) <= leps) lo = mid;
-          else hi = mid;
-        }
-        load_cell(c, i0, lo);
-        elo = mix(c.e, 0);
-        ehi = mix(c.e, 1);
       }
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (node(mid) <= leps) lo = mid;
+        else hi = mid;
+      }
+      if (lo != c.i1) load_cell(c, i0, lo);
+      elo = mix(c.e, 0);
+      ehi = mix(c.e, 1);
     }
     double f; // log T weight in the cell
     if (c.i1 == 0 && leps <= elo) { // at or below the table's lowest T

@@ -136,7 +136,8 @@ _eosio = None
 class asx_eos_host_table(C.Structure):
     _fields_ = [("n", C.c_int32 * 3), ("data", C.POINTER(C.c_double)),
                 ("axis", C.POINTER(C.c_double) * 3), ("energy_shift", C.c_double),
-                ("eps_min", C.c_double), ("eps_max", C.c_double)]
+                ("eps_min", C.c_double), ("eps_max", C.c_double),
+                ("eps_grows_with_T", C.c_int32), ("pad0", C.c_int32)]
 
 
 def eosio():

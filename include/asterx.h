@@ -116,6 +116,13 @@ typedef struct asx_eos_table_s {
   /* host copies of axis[d][0], axis[d][1] - axis[d][0], axis[d][n[d]-1]
    * (the library does not read the device table from the host) */
   double x_lo[3], x_step[3], x_hi[3];
+  /* 1: log(eps + energy_shift) grows by more than 1e-12 from every T node to
+   * the next, at every (log rho, Ye) node, so that one T has a given eps and
+   * con2prim may look for it from the zone's previous temperature.  Any
+   * other value (0 where it is not known): every temperature solve bisects
+   * the whole T axis, as asx_eos_from_rho_eps does, several times slower. */
+  int32_t eps_grows_with_T;
+  int32_t pad0;
 } asx_eos_table;
 
 typedef struct {

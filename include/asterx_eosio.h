@@ -24,14 +24,16 @@ extern "C" {
  * c_s^2 (code units) and the entropy per baryon; axis[0] = log rho and
  * axis[1] = log T (natural logs, code units, T in MeV), axis[2] = Ye;
  * eps_min / eps_max = min and max of exp(log(eps + shift)) - shift over the
- * nodes, the minimum floored at 1e-15.  Arrays owned by the library until
- * asx_eos_host_table_free. */
+ * nodes, the minimum floored at 1e-15; eps_grows_with_T as asx_eos_table's.
+ * Arrays owned by the library until asx_eos_host_table_free. */
 typedef struct {
   int32_t n[3];
   double *data;
   double *axis[3];
   double energy_shift;
   double eps_min, eps_max;
+  int32_t eps_grows_with_T;
+  int32_t pad0;
 } asx_eos_host_table;
 
 /* EOSX's StellarCollapse reader (eos_3p_tabulated3d.hxx:53-193): the

@@ -100,3 +100,22 @@ def test_reader_refuses_bad_files(tmp_path):
     write_stellarcollapse(path, ds)
     assert L.asx_eos_read_stellarcollapse(path.encode(), C.byref(t)) == 3
     assert L.asx_eos_read_stellarcollapse(None, C.byref(t)) == 1
+
+
+@pytest.mark.parametrize("node", [None, (0, 0, 0), (8, 15, 22), (4, 7, 11)])
+def test_growth_with_temperature(tmp_path, node):
+    """Reader and descriptor say whether log(eps + shift) grows from every T
+    node to the next; one node that does not is found wherever it lies."""
+    ds, _ = _datasets()
+    if node is not None:
+        k, j, i = node
+        ds["logenergy"] = ds["logenergy"].copy()
+        ds["logenergy"][k, j, i] = ds["logenergy"][k, j + 1, i] - 1e-14
+    path = str(tmp_path / "t.h5")
+    write_stellarcollapse(path, ds)
+    L, t = lib.eosio(), lib.asx_eos_host_table()
+    assert L.asx_eos_read_stellarcollapse(path.encode(), C.byref(t)) == 0
+    assert t.eps_grows_with_T == (node is None)
+    L.asx_eos_host_table_free(C.byref(t))
+    host = tabeos.Table(tabeos.read_stellarcollapse(path), device=None)
+    assert host.desc.eps_grows_with_T == (node is None)
