@@ -415,12 +415,14 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
   else if (x0 > 1e20) x0 = xo0;
   double dx0 = 1., df = 1., f = 1.;
   bool conv = false;
-  // What a step costs is its divisions.  The residuals r0 and r1 keep the
-  // reference's roundings (1/Z and the quotient by Gamma are rounded
-  // quotients); the derivatives, whose rounding the next step corrects, take
-  // the factor (Gamma - 1)/Gamma and reciprocals good to about a unit in the
-  // last place, and the step is compared with tol |Z| instead of divided by
-  // Z: seven divisions a step become two reciprocals and an estimate.
+  // What a step costs is its divisions.  Only the residual's quotient by
+  // Gamma is rounded as the reference rounds it; 1/Z (in the residuals too),
+  // 1/det and 1/sqrt(1 - v^2) are reciprocals good to about a unit in the
+  // last place, the derivatives take the factor (Gamma - 1)/Gamma, and the
+  // step is compared with tol |Z| instead of divided by Z: seven divisions a
+  // step become three such reciprocals.  A Jacobian that is singular
+  // makes the step infinite, as by the reference's division, and the limits
+  // below put Z back and v^2 inside its range; 1 - v^2 is at least 2^-53.
   const Divisor dG(G);
   const double gfac = (G - 1.0) * dG.r;
   int k;
@@ -444,7 +446,7 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
     const double detjac =
         (Bsq + Z) * (j10 * (Bsq + Z) +
                      (Bsq - 2.0 * dPdvsq) * (BiSi * BiSi * invZ * invZ + Vsq * Z) * invZ);
-    const double detjac_inv = rcp_normal(detjac);
+    const double detjac_inv = rcp_any(detjac);
     dx0 = -(j11 * r0 - j01 * r1) * detjac_inv;
     const double dx1 = -(-j10 * r0 + j00 * r1) * detjac_inv;
     df = -r0 * r0 - r1 * r1;

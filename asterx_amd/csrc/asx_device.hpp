@@ -258,6 +258,9 @@ ASX_DEV double rcp_normal(double x) {
   r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
   return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
 }
+// The same for every x: the Newton steps turn the estimate for a zero or an
+// infinity into NaN, which the division's own last instruction puts right.
+ASX_DEV double rcp_any(double x) { return __builtin_amdgcn_div_fixup(rcp_normal(x), x, 1.0); }
 
 // WENO-Z face values of the centre cell (ReconX/src/wenoz.hxx:23-99).
 // Same smoothness indicators, weights and stencils; the nonlinear weights

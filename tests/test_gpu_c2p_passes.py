@@ -129,3 +129,25 @@ def test_table_patch():
     for k in outs:
         a = np.tile(got[0][k], [-(-n[2 - q] // n0[2 - q]) for q in range(3)])
         assert np.array_equal(got[1][k], a[:n[2], :n[1], :n[0]], equal_nan=True), k
+
+
+@pytest.mark.parametrize("nz", [1, ONE_PASS + 1])
+def test_singular_newton_step(nz):
+    """Gamma = 4, D = 5, v^2 = 3/4 and Z = 18 make the Jacobian of Noble's
+    first step exactly zero: the step is infinite, Z is put back and the
+    iteration goes on, to the root, as in the oracle."""
+    g = np.zeros((6, 1))
+    g[[0, 3, 5]] = 1.0
+    cons = np.array([[5.0, 3.0, 0, 0, 4.0, 0, 0, 0]]).T
+    seed = np.array([[2.5, 0.2, 0.5, 0.5, 0.5]]).T
+    par = abi.params(gl_gamma=4.0, eps_max=1e8, rho_max=1e8, rho_abs_min=1e-12, vw_lim=1e3,
+                     B_lim=1e3, c2p_prime="Noble", c2p_second="None", max_iter=60)
+    cons, g, seed = (np.ascontiguousarray(np.repeat(a, nz, axis=1)) for a in (cons, g, seed))
+    prim, flag, it = np.zeros((8, nz)), np.zeros(nz), np.zeros(nz, dtype=np.int32)
+    abi.check("orc_c2p_batch", oracle.lib().orc_c2p_batch(
+        nz, cons.ctypes.data, g.ctypes.data, seed.ctypes.data, prim.ctypes.data,
+        flag.ctypes.data, it.ctypes.data, C.byref(par)))
+    assert (flag == 1).all()
+    got, gflag, git = _solve(par, cons, g, seed)
+    assert np.array_equal(gflag, flag) and np.array_equal(git, it)
+    assert rel_err(got, prim) <= 1e-12
