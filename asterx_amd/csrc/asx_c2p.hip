@@ -155,11 +155,11 @@ __global__ __launch_bounds__(256) void k_c2p_patches(const KPatch *__restrict__ 
 
 // Independent zones (layout of asx_c2p_batch in include/asterx.h) in two
 // passes without scratch memory: every zone through the primary solver, which
-// alone sets the register budget (152 VGPRs and 3 waves per SIMD for Noble,
-// 208 and 2 for the full chain); a zone it fails gets the flag kZoneFailed,
+// alone sets the register budget (124 VGPRs for Noble and 114 for Palenzuela,
+// 4 waves per SIMD; 241 and 2 for the full chain); a zone it fails gets the flag kZoneFailed,
 // which the second pass looks for.  Bound by the latency of the Newton
 // steps' dependent square roots and reciprocals: 4 000 037 zones from the
-// previous step's primitives 0.770 -> 0.497 ms (0.13 of them the second pass).
+// previous step's primitives 0.770 -> 0.470 ms (0.13 of them the second pass).
 constexpr double kZoneFailed = -1.0;
 template <int PRIME>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))

@@ -307,32 +307,33 @@ ASX_DEV void vel_from_Z(double Z, double W, double Bsq, double BiSi, const Cons 
                         const Sym3 &gup, const Sym3 &glo, bool use_z, Prim &pv) {
   const double *m = cv.mom;
   const double *B = cv.dB;
+  const double f = use_z ? W : 1.0; // z = W v
+  const double a[3] = {f * (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]),
+                       f * (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]),
+                       f * (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2])};
+  double u[3];
+  auto over = [&](const auto &zb, const auto &zzb) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      u[i] = a[i] / zb;
+      u[i] += f * BiSi * B[i] / zzb;
+    }
+  };
   const Divisor zb(Z + Bsq), zzb(Z * (Z + Bsq));
+  if (zb.holds() && zzb.holds()) over(zb, zzb);
+  else over(zb.d, zzb.d);
   if (use_z) {
-    double zx = W * (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / zb;
-    zx += W * BiSi * B[0] / zzb;
-    double zy = W * (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / zb;
-    zy += W * BiSi * B[1] / zzb;
-    double zz = W * (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / zb;
-    zz += W * BiSi * B[2] / zzb;
-    const double zxd = glo.xx * zx + glo.xy * zy + glo.xz * zz;
-    const double zyd = glo.xy * zx + glo.yy * zy + glo.yz * zz;
-    const double zzd = glo.xz * zx + glo.yz * zy + glo.zz * zz;
-    const double lor = sqrt(1.0 + (zx * zxd + zy * zyd + zz * zzd));
-    const Divisor dl(lor);
-    pv.vel[0] = zx / dl;
-    pv.vel[1] = zy / dl;
-    pv.vel[2] = zz / dl;
-    pv.w_lor = lor;
-  } else {
-    pv.vel[0] = (gup.xx * m[0] + gup.xy * m[1] + gup.xz * m[2]) / zb;
-    pv.vel[0] += BiSi * B[0] / zzb;
-    pv.vel[1] = (gup.xy * m[0] + gup.yy * m[1] + gup.yz * m[2]) / zb;
-    pv.vel[1] += BiSi * B[1] / zzb;
-    pv.vel[2] = (gup.xz * m[0] + gup.yz * m[1] + gup.zz * m[2]) / zb;
-    pv.vel[2] += BiSi * B[2] / zzb;
-    pv.w_lor = W;
+    double u_low[3];
+    lower(glo, u, u_low);
+    W = sqrt(1.0 + (u[0] * u_low[0] + u[1] * u_low[1] + u[2] * u_low[2]));
+    const Divisor dl(W);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) u[i] /= dl;
   }
+  pv.vel[0] = u[0];
+  pv.vel[1] = u[1];
+  pv.vel[2] = u[2];
+  pv.w_lor = W;
 }
 
 // Noble 2D Newton on (Z, v^2), c2p_2DNoble.hxx:275-594.  z0/v0 (if >= 0)

@@ -15,9 +15,11 @@
 
 #include "asterx.h"
 
+#define ASX_DEV __device__ __forceinline__
+#include "asx_quotient.hpp"
+
 namespace asx {
 
-#define ASX_DEV __device__ __forceinline__
 // The library builds with -ffp-contract=off so that con2prim and the
 // reconstruction (whose limiter branches compare computed values) evaluate
 // their expressions exactly as written.  The smooth arithmetic after the
@@ -101,22 +103,6 @@ ASX_DEV int xcd_tile(int w, int nb) {
   return (rem == 0 || x < rem) ? x * per + l : rem * per + (x - rem) * (per - 1) + l;
 }
 
-// Quotients by one divisor: x / d from d's correctly rounded reciprocal with
-// the remainder of the first product added back (Markstein's sequence).  The
-// result is the rounded quotient, the same bits as a division, in six
-// instructions instead of about a dozen with a quarter-rate one among them;
-// zeros, infinities and NaN in x or d give what a division gives (but for
-// the sign of a zero), and only a subnormal remainder may cost the last bit.
-struct Divisor {
-  double d, r;
-  ASX_DEV explicit Divisor(double x) : d(x), r(1.0 / x) {}
-};
-ASX_DEV double operator/(double x, const Divisor &v) {
-  const double q = x * v.r, e = __builtin_fma(-v.d, q, x);
-  return e == e ? __builtin_fma(e, v.r, q) : q;
-}
-ASX_DEV double &operator/=(double &x, const Divisor &v) { return x = x / v; }
-
 struct Sym3 {
   double xx, xy, xz, yy, yz, zz;
   ASX_DEV double operator()(int i, int j) const {
@@ -131,10 +117,13 @@ ASX_DEV double det3(const Sym3 &g) {
          g.xx * pow2(g.yz) - g.zz * pow2(g.xy);
 }
 ASX_DEV Sym3 inv3(const Sym3 &g, double det) {
+  auto over = [&](const auto &d) {
+    return Sym3{(g.yy * g.zz - pow2(g.yz)) / d, (g.xz * g.yz - g.xy * g.zz) / d,
+                (g.xy * g.yz - g.xz * g.yy) / d, (g.xx * g.zz - pow2(g.xz)) / d,
+                (g.xy * g.xz - g.xx * g.yz) / d, (g.xx * g.yy - pow2(g.xy)) / d};
+  };
   const Divisor d(det);
-  return Sym3{(g.yy * g.zz - pow2(g.yz)) / d, (g.xz * g.yz - g.xy * g.zz) / d,
-              (g.xy * g.yz - g.xz * g.yy) / d, (g.xx * g.zz - pow2(g.xz)) / d,
-              (g.xy * g.xz - g.xx * g.yz) / d, (g.xx * g.yy - pow2(g.xy)) / d};
+  return d.holds() ? over(d) : over(det);
 }
 ASX_DEV void lower(const Sym3 &g, const double v[3], double o[3]) {
   o[0] = 0.0 + g.xx * v[0] + g.xy * v[1] + g.xz * v[2];
@@ -249,18 +238,6 @@ struct Diff4 {
   ASX_DEV Diff4(double gImm, double gIm, double gI, double gIp, double gIpp)
       : e0(gIm - gImm), e1(gI - gIm), e2(gIp - gI), e3(gIpp - gIp) {}
 };
-
-// 1 / x for a normal x whose reciprocal is normal too, within about one unit
-// in the last place: the hardware estimate and two Newton steps, without the
-// scaling and the fix-ups of a division that works over the whole range.
-ASX_DEV double rcp_normal(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-}
-// The same for every x: the Newton steps turn the estimate for a zero or an
-// infinity into NaN, which the division's own last instruction puts right.
-ASX_DEV double rcp_any(double x) { return __builtin_amdgcn_div_fixup(rcp_normal(x), x, 1.0); }
 
 // WENO-Z face values of the centre cell (ReconX/src/wenoz.hxx:23-99).
 // Same smoothness indicators, weights and stencils; the nonlinear weights
