@@ -77,6 +77,13 @@ template <bool WIDE> ASX_DEV void load_fence() {
   }
 }
 
+// Keeps a sum's first value out of the fused multiply-adds of what is added
+// to it, as the loop that adds it does where it is not unrolled: both forms
+// of the update then round alike (no instruction).
+template <bool WIDE> ASX_DEV void round_here(double &x) {
+  if constexpr (WIDE) asm("" : "+v"(x));
+}
+
 // Gradient of vertex field g at cell (vertex base o), order 2 or 4.
 template <int ORD, bool WIDE>
 ASX_DEV void cell_grad(const KPatch &P, const double *g, int o, double out[3]) {
@@ -184,6 +191,7 @@ ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
   //   tau_S = -T^00 beta.d(alpha) - t0.d(alpha) + sum_{a<=b} K_ab D_ab,
   //   D_ab = w_ab (T^00 beta^a beta^b + T^ab) + 2 (t0^a beta^b + t0^b beta^a) / (1 + [a==b])
   double tau_source = -t00 * dot3(beta, d_alp) - dot3(t0, d_alp);
+  round_here<WIDE>(tau_source);
   {
     double dk[6];
 #pragma unroll
@@ -206,7 +214,10 @@ ASX_DEV void source_cell(const KPatch &P, int i, int j, int k, const RhsArgs &A,
   }
   double ms[3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) ms[d] = -(t00 * alp) * d_alp[d];
+  for (int d = 0; d < 3; ++d) {
+    ms[d] = -(t00 * alp) * d_alp[d];
+    round_here<WIDE>(ms[d]);
+  }
   // the derivative pass re-reads the metric (cache hits) rather than keeping
   // 80 corner values live across the stress-energy computation
   // coefficient of each derivative: beta^x, beta^y, beta^z, then g_ab
