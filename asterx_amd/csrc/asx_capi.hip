@@ -2412,7 +2412,7 @@ asx_status plan_capture(asx_batch *b) {
 }
 
 // The three stages' argument blocks of the persistent form (built once):
-// launch lists of the persistent kernel's fixed shapes (face variant 0 of
+// launch lists of the persistent kernel's fixed shapes (face variant 8 of
 // every direction, update tiles of kPersistUpdateTile = variant 1).
 asx_status plan_persist_prepare(asx_batch *b) {
   if (b->pargs) return ASX_OK;
@@ -2436,7 +2436,7 @@ asx_status plan_persist_prepare(asx_batch *b) {
   PersistArgs a;
   std::memset(&a, 0, sizeof(a));
   for (int d = 0; d < 3; ++d)
-    if (!list(BK_FACE + d, 0, a.face[d])) return st;
+    if (!list(BK_FACE + d, 8, a.face[d])) return st;
   if (!list(BK_BC, 0, a.bc) || !list(BK_AUX, 0, a.aux) || !list(BK_UPDATE, 1, a.update) || !list(BK_C2P, 0, a.c2p))
     return st;
   a.A = plan_flux_args(&par);

@@ -495,20 +495,17 @@ ASX_DEV void face_flux(const KPatch &P, const FluxArgs &A, int i, int j, int k,
   }
 }
 
-// Face tile shapes (x, y, z work-items; 256 per block), variant V of the
-// faces normal to D.  The extent along D is one cell more than the faces the
-// tile produces.
+// Face tile shapes (x, y, z work-items; 256 per block), variant V >= 1 of the
+// faces normal to D (variant 0: face_shape()).  The extent along D is one cell
+// more than the faces the tile produces.
 template <int X_, int Y_, int Z_> struct Tile3 {
   static constexpr int X = X_, Y = Y_, Z = Z_;
 };
 template <int D, int V> struct FaceTileT;
-template <> struct FaceTileT<0, 0> { using T = Tile3<64, 4, 1>; };
 template <> struct FaceTileT<0, 1> { using T = Tile3<64, 2, 2>; };
 template <> struct FaceTileT<0, 2> { using T = Tile3<32, 4, 2>; };
-template <> struct FaceTileT<1, 0> { using T = Tile3<16, 16, 1>; };
 template <> struct FaceTileT<1, 1> { using T = Tile3<32, 8, 1>; };
 template <> struct FaceTileT<1, 2> { using T = Tile3<16, 8, 2>; };
-template <> struct FaceTileT<2, 0> { using T = Tile3<16, 1, 16>; };
 template <> struct FaceTileT<2, 1> { using T = Tile3<32, 1, 8>; };
 template <> struct FaceTileT<2, 2> { using T = Tile3<16, 2, 8>; };
 // narrower rows: fewer idle work-items on extents such as n + 2
@@ -528,7 +525,12 @@ template <> struct FaceTileT<1, 7> { using T = Tile3<8, 8, 4>; };
 template <> struct FaceTileT<2, 5> { using T = Tile3<16, 2, 8>; };
 template <> struct FaceTileT<2, 6> { using T = Tile3<8, 2, 16>; };
 template <> struct FaceTileT<2, 7> { using T = Tile3<8, 4, 8>; };
-constexpr int kFaceStagedVariant = 5; // variants from here on stage the metric
+constexpr bool face_staged(int v) { return v >= 5 && v <= 7; }
+// long rows in x and deep ones in z, for boxes that fill them (the shapes of
+// the persistent stage); in y the library's choice
+template <> struct FaceTileT<0, 8> { using T = Tile3<64, 4, 1>; };
+template <> struct FaceTileT<1, 8> { using T = Tile3<16, 16, 1>; };
+template <> struct FaceTileT<2, 8> { using T = Tile3<16, 1, 16>; };
 template <int D, int V> using FaceTile = typename FaceTileT<D, V>::T;
 
 // LDS of a face tile: the high side of every cell, handed to the next cell
@@ -545,7 +547,7 @@ struct FaceLDS {
 // per work-item instead of 40) at the start of the tile, written to LDS
 // after the reconstruction and summed after the hand-over barrier, so the
 // metric's latency overlaps the reconstruction's.  Only for tile shapes
-// (variants kFaceStagedVariant and up), whose box leaves room for three
+// (face_staged), whose box leaves room for three
 // workgroups per CU (<= 33 KB beside the hand-over); the others load the
 // metric per face.
 template <int D, int V> struct MetricBox {
@@ -560,7 +562,7 @@ template <int D, int V> struct MetricBox {
   static constexpr int BXS = PAIR ? BXE : BX; // LDS row stride
   static constexpr int VB = BXS * BY * BZ, N = 10 * VB;
   static constexpr int NV = PAIR ? (VB / 2 + 255) / 256 : (VB + 255) / 256;
-  static constexpr bool ok = V >= kFaceStagedVariant;
+  static constexpr bool ok = face_staged(V);
   static_assert(!ok || N * 8 <= 33 * 1024, "staged metric box too large for 3 workgroups per CU");
 };
 

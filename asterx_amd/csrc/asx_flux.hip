@@ -38,7 +38,7 @@ void k_face(KPatch P, FluxArgs A, int ntx, int nty, int ntz) {
 // tiles are narrow, the 16 x 16 rows of per-face loads are as fast.
 template <int M, bool TAB> struct FaceShapes {
   static constexpr bool staged = TAB || M == ASX_RECON_WENOZ || M == ASX_RECON_MP5;
-  static constexpr int X = staged ? 5 : 4, Y = 0, Z = staged ? 5 : 3;
+  static constexpr int X = staged ? 5 : 4, Y = 8, Z = staged ? 5 : 3;
 };
 int face_shape(int d, int method, bool tab) {
   using S = FaceShapes<ASX_RECON_WENOZ, false>;
@@ -220,7 +220,7 @@ static hipError_t launch_flux_d(const KPatch &P, const FluxArgs &A, int method, 
   case 5: return launch_flux_dv<D, 5>(P, A, method, s, tab);
   case 6: return launch_flux_dv<D, 6>(P, A, method, s, tab);
   case 7: return launch_flux_dv<D, 7>(P, A, method, s, tab);
-  default: return launch_flux_dv<D, D == 1 ? 0 : 5>(P, A, method, s, tab);
+  default: return launch_flux_dv<D, 8>(P, A, method, s, tab);
   }
 }
 
@@ -407,7 +407,7 @@ static void launch_face_batch_d(const KPatch *tab, const FluxArgs &A, const Batc
   case 5: launch_face_batch_dv<D, 5>(tab, A, box, map, nmap, method, s); break;
   case 6: launch_face_batch_dv<D, 6>(tab, A, box, map, nmap, method, s); break;
   case 7: launch_face_batch_dv<D, 7>(tab, A, box, map, nmap, method, s); break;
-  default: launch_face_batch_dv<D, D == 1 ? 0 : 5>(tab, A, box, map, nmap, method, s); break;
+  default: launch_face_batch_dv<D, 8>(tab, A, box, map, nmap, method, s); break;
   }
 }
 
@@ -426,7 +426,7 @@ template <int D> static void face_ext_d(int variant, int ex[3]) {
   case 5: face_ext<D, 5>(ex); break;
   case 6: face_ext<D, 6>(ex); break;
   case 7: face_ext<D, 7>(ex); break;
-  default: face_ext<D, 0>(ex); break;
+  default: face_ext<D, 8>(ex); break;
   }
 }
 void face_tile_extent(int d, int variant, int ex[3]) {

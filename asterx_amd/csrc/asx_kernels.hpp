@@ -95,7 +95,7 @@ template <int TX, int TY, int TZ, int YS> struct TileGridBand {
 // Launch-shape variants of the tunable kernels (selected per call; see
 // asx_set_variant / asx_autotune_substep in the C ABI).
 constexpr int kUpdateVariants = 7;
-constexpr int kFaceVariants = 8; // 5-7 stage the tile's vertex metric in LDS
+constexpr int kFaceVariants = 9; // 5-7 stage the tile's vertex metric in LDS
 constexpr int kTmunuVariants = 9;
 
 // Batched launches over many patches: the workgroups of one launch are
@@ -384,7 +384,7 @@ hipError_t launch_con2prim_patches(const KPatch *tab, const IdealGas &eos, const
                                    const BatchRef *map, int nmap, hipStream_t s);
 // A whole SSPRK3 stage of a batch as one persistent cooperative launch
 // (asx_plan.hip): the launch lists of each phase and everything the phases
-// read, in device memory.  Faces use tile variant 0 of every direction, the
+// read, in device memory.  Faces use tile variant 8 of every direction, the
 // update 32x4x2 tiles (kPersistUpdateTile), con2prim Noble as the primary.
 struct BatchList {
   const BatchBox *box;

@@ -52,9 +52,9 @@ ASX_ITEM void face_item(const PersistArgs &S, int d, int q, FaceLDS &L) {
   const BatchRef ref = S.face[d].map[q];
   const BatchBox &bb = S.face[d].box[ref.pid];
   const KPatch &P = S.T[ref.pid];
-  if (d == 0) face_tile<0, M, 0>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
-  else if (d == 1) face_tile<1, M, 0>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
-  else face_tile<2, M, 0>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
+  if (d == 0) face_tile<0, M, 8>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
+  else if (d == 1) face_tile<1, M, 8>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
+  else face_tile<2, M, 8>(P, S.A, bb.lo, bb.cnt, ref.chunk, bb.nt[0], bb.nt[1], L);
 }
 
 ASX_ITEM void aux_item(const PersistArgs &S, int q) {

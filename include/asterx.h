@@ -365,7 +365,8 @@ asx_status asx_poison_check(const asx_patch *patch, int32_t slot, const int32_t 
  * by the fp32 summation order only.  The choice is per device (default 0).
  * Variant 0 of a face class leaves the shape to the library; while all three
  * are 0, one launch computes the faces of every direction and the vertex
- * auxiliaries of a patch.  asx_autotune_substep
+ * auxiliaries of a patch.  Face variant 8 has the longest rows (64 x 4 x 1
+ * work-items in x, 16 x 16 x 1 in y, 16 x 1 x 16 in z).  asx_autotune_substep
  * runs asx_substep with the given arguments once untimed and `reps` times
  * timed for every variant, keeps the fastest per kernel class (or the one
  * launch, where that is faster), and leaves the caller's timing state as it
@@ -777,7 +778,7 @@ asx_status asx_batch_stage(asx_batch *plan, int32_t stage, void *stream);
  * workgroups walk every phase over every patch (faces and aux, update,
  * state fill, con2prim, queued zones, primitive fill) with grid-wide
  * barriers between phases, every workgroup resident for the whole stage;
- * it uses fixed launch shapes (face variant 0, update variant 1) and is
+ * it uses fixed launch shapes (face variant 8, update variant 1) and is
  * built for PPM, WENO-Z and MP5 with Noble as the primary solver and
  * without caller dB_stag (ASX_ERR_UNSUPPORTED otherwise).  All three modes
  * give the same results bit for bit.  Other values: ASX_ERR_PARAM. */

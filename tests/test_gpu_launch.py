@@ -86,6 +86,35 @@ def test_faces_in_one_launch(n, recon, halo):
         assert np.array_equal(got[0][m], got[1][m]), m
 
 
+@pytest.mark.parametrize("n", [(62, 4, 3), (64, 17, 16), (130, 3, 33)])
+@pytest.mark.parametrize("recon", ["wenoz", "ppm"])
+def test_long_row_faces(n, recon):
+    """The tiles of long rows (variant 8: 64 x 4 x 1 in x, 16 x 1 x 16 in z) at
+    and beside whole rows, one direction at a time, against the one launch."""
+    torch = _torch()
+    L = _lib()
+    par = abi.params(reconstruction_method=recon, flux_type="HLLE", loworder_method="minmod")
+    kcs = [abi.KCLASS["face_" + c] for c in "xyz"]
+    got = []
+    try:
+        for pick in (None, 0, 1, 2):
+            for d, kc in enumerate(kcs):
+                abi.check("asx_set_variant", L.asx_set_variant(kc, 8 if d == pick else 0))
+            p = make_state(n=n, curved=True, zero_entropy_block=True).to("cuda")
+            for name in abi.FLUX:
+                p[name].fill_(0.0)
+            abi.check("asx_fluxes", L.asx_fluxes(C.byref(p.struct()), C.byref(par), 1, None,
+                                                 None))
+            torch.cuda.synchronize()
+            got.append({m: p.numpy(m) for m in abi.FLUX})
+    finally:
+        for kc in kcs:
+            abi.check("asx_set_variant", L.asx_set_variant(kc, 0))
+    for g in got[1:]:
+        for m in abi.FLUX:
+            assert np.array_equal(got[0][m], g[m]), m
+
+
 @pytest.mark.parametrize("order", [2, 4])
 @pytest.mark.parametrize("n,nz", [((160, 90, 130), 9), ((40, 20, 60), 1), ((5, 3, 17), 4)])
 def test_tmunu_runs(order, n, nz):
