@@ -62,6 +62,17 @@ class Evolution:
         self.b.bc_fill_many(ps, [abi.SLOT[n] for n in names if n in self.p],
                             self.bc)
 
+    # The SYNC after one of several calls on the patch's struct ps; returns
+    # the struct for the next call.  A program's own sync (an exchange with
+    # other patches) may put other arrays in the patch, so the struct is built
+    # anew after it.
+    def _sync(self, names, ps):
+        if getattr(self.sync, "__func__", None) is Evolution.sync:
+            self.sync(names, ps)
+            return ps
+        self.sync(names)
+        return self.p.struct()
+
     # AsterX_InitialGroup (check_prims is given: it is initial-data only)
     def initial(self, check_prims):
         p, b = self.p, self.b
@@ -86,22 +97,22 @@ class Evolution:
             return
         ps = p.struct()
         b.fluxes(ps, par, 0)
-        self.sync(SYNC_FLUXES + (SYNC_UCT if self.uct else []), ps)
+        ps = self._sync(SYNC_FLUXES + (SYNC_UCT if self.uct else []), ps)
         b.source_terms(ps, par)
-        self.sync(SYNC_RHS_HYDRO, ps)
+        ps = self._sync(SYNC_RHS_HYDRO, ps)
         b.rhs(ps, par)
-        self.sync(SYNC_RHS_HYDRO + SYNC_RHS_EM, ps)
+        self._sync(SYNC_RHS_HYDRO + SYNC_RHS_EM, ps)
 
     def poststep(self):
         p, b = self.p, self.b
         ps = p.struct()
-        self.sync(abi.STATE, ps)
+        ps = self._sync(abi.STATE, ps)
         b.bstag_from_A(ps)
-        self.sync(abi.DBSTAG, ps)
+        ps = self._sync(abi.DBSTAG, ps)
         b.dB_from_bstag(ps)
-        self.sync(abi.DB, ps)
+        ps = self._sync(abi.DB, ps)
         b.con2prim(ps, self.par)
-        self.sync(SYNC_C2P, ps)
+        self._sync(SYNC_C2P, ps)
         if self.with_tmunu:
             self.tmunu()
 
