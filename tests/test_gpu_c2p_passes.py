@@ -91,26 +91,31 @@ def test_patch_with_failures(n):
         assert rel_err(d.numpy(name)[sl], h.numpy(name)[sl]) <= 1e-9, name
 
 
-def test_table_patch():
+@pytest.mark.parametrize("second", ["None", "Palenzuela"])
+@pytest.mark.parametrize("n", [(64, 33, 32), (64, 32, 45)])
+def test_table_patch(n, second):
     """Past the table's line (65536 zones) the two passes, before it one: a
-    patch tiled from a small one, zone by zone the same bits."""
+    patch tiled from a small one, zone by zone the same bits, and the counters
+    of the same zones.  With a backup the zones that the primary failed go
+    through the queue, without one they end in the first pass."""
     torch = _torch()
     from asterx_amd import lib, tabeos
     from asterx_amd.patch import Patch
     table = tabeos.build()
-    kw = dict(c2p_prime="Palenzuela", c2p_second="None", use_temperature=1, use_press_atmo=0,
+    kw = dict(c2p_prime="Palenzuela", c2p_second=second, use_temperature=1, use_press_atmo=0,
               thermal_eos_atmo=1, t_atmo=0.01, Ye_atmo=0.3, c2p_tol=1e-10, max_iter=100,
               vw_lim=1e3, B_lim=1e3, ye_min=0.035, ye_max=0.55, rho_abs_min=1e-12)
     htab, dtab = tabeos.Table(table, device=None), tabeos.Table(table, device="cuda")
-    n0, n = (16, 16, 15), (64, 33, 32)
+    n0 = (16, 16, 15)
     par = dtab.attach(abi.params(**kw))
     src = make_state(n=n0, curved=False, table_par=htab.attach(abi.params(**kw)))
     src["dens"][5, 6, 7] = 1e-25  # atmosphere
     src["tau"][4::4, 5::5, 6::3] = -1.0  # floored
     src["dens"][9, 9, 9] = np.nan
+    src["dBy"][3::5, 7::6, 5::4] = 1e4  # beyond B_lim: the primary fails
     cells = abi.CONS + abi.DB + abi.SAVED + ["temperature"]
     outs = abi.PRIMS + abi.CONS + abi.DB + abi.SAVED + abi.ZS + ["con2prim_flag"]
-    got = []
+    got, cnts = [], []
     for m in (n0, n):
         d = Patch(m, 3, src.x0, src.dx, slots=set(abi.ADM + cells + outs), device="cuda")
         for name in ("alp", "gxx", "gyy", "gzz"):
@@ -121,14 +126,23 @@ def test_table_patch():
             full = np.zeros(d.shape(name))
             full[d.interior(name)] = a[:m[2], :m[1], :m[0]]
             d[name] = full
+        cnt = abi.asx_counters()
         abi.check("asx_con2prim", lib.lib().asx_con2prim(C.byref(d.struct()), C.byref(par),
-                                                         None, None))
+                                                         C.byref(cnt), None))
         torch.cuda.synchronize()
         got.append({k: d.numpy(k)[d.interior(k)] for k in outs})
-    assert len(np.unique(got[0]["con2prim_flag"])) >= 2
+        cnts.append((list(cnt.c2p_flags), list(cnt.c2p_iters)))
+        fl = got[-1]["con2prim_flag"].astype(int).ravel()
+        assert list(np.bincount(fl, minlength=7)) == cnts[-1][0]
+        assert sum(cnts[-1][1]) == fl.size
+    flags = cnts[1][0]
+    assert flags[6] > 300 and flags[1] > 10000 and sum(x > 0 for x in flags) >= 3
     for k in outs:
         a = np.tile(got[0][k], [-(-n[2 - q] // n0[2 - q]) for q in range(3)])
         assert np.array_equal(got[1][k], a[:n[2], :n[1], :n[0]], equal_nan=True), k
+    if all(n[q] % n0[q] == 0 for q in range(3)):
+        times = int(np.prod(n) // np.prod(n0))
+        assert cnts[1][1] == [times * x for x in cnts[0][1]]
 
 
 @pytest.mark.parametrize("nz", [1, ONE_PASS + 1])
