@@ -92,12 +92,11 @@ void k_update_all(KPatch P, Box B, G_ G, RhsArgs A, StatePtrs u0, StatePtrs out,
 
 // One wavefront per workgroup and SIMD: see load_fence<WIDE>.
 using WideTiles = TileGrid<16, 2, 2>;
-template <int ORD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void k_update_wide(KPatch P, Box B, WideTiles G, RhsArgs A, StatePtrs u0, StatePtrs out, Comb cb) {
   int i, j, k;
   if (!G.point(B, i, j, k)) return;
-  update_point<ORD, true>(P, i, j, k, A, u0, out, cb);
+  update_point<2, true>(P, i, j, k, A, u0, out, cb);
 }
 
 template <int ORD, int TX, int TY, int TZ>
@@ -271,15 +270,15 @@ hipError_t launch_update(const KPatch &P, const RhsArgs &A, const StatePtrs &u0,
                          int variant, hipStream_t s) {
   const Comb cb{c0, c1, c2};
   const Box b = interior_box(P, 7);
-  // Up to one wavefront a SIMD (256 CUs of 4): every load in flight (22 x 17 x
-  // 13: 18.1 us with the fences, 14.5 without; substep of 40 x 37 x 31 43 -> 38
-  // us, but of 50^3, three wavefronts a SIMD, 70 -> 85)
+  // Up to one wavefront a SIMD (256 CUs of 4): every load in flight (8^3 21.9 us
+  // with the fences, 16.7 without; 22 x 17 x 13 19.3 / 16.5; 31^3 21.9 / 19.8; 63
+  // x 31 x 30 23.5 / 22.8; substep of 50^3, three wavefronts a SIMD, 70 / 85).
+  // Not at order 4, whose 432 corner and stencil values a derivative pass would
+  // hold do not fit the registers: 22 x 17 x 13 23 us with the fences, 44 without,
+  // 31^3 27 / 73.
   const WideTiles w = WideTiles::make(b);
-  if (variant == 0 && (int64_t)w.ntx * w.nty * w.ntz <= 1024) {
-    if (A.fd_order == 4)
-      hipLaunchKernelGGL(k_update_wide<4>, w.grid(), dim3(64), 0, s, P, b, w, A, u0, out, cb);
-    else
-      hipLaunchKernelGGL(k_update_wide<2>, w.grid(), dim3(64), 0, s, P, b, w, A, u0, out, cb);
+  if (variant == 0 && A.fd_order != 4 && (int64_t)w.ntx * w.nty * w.ntz <= 1024) {
+    hipLaunchKernelGGL(k_update_wide, w.grid(), dim3(64), 0, s, P, b, w, A, u0, out, cb);
     return hipGetLastError();
   }
   if (A.fd_order == 4)
