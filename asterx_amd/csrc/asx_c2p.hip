@@ -105,7 +105,9 @@ __global__ __launch_bounds__(256) void k_c2p_rest(KPatch P, Box B, E eos, C2PArg
 // atmosphere.  A second pass over queued zones repeats the failed primary in
 // a few wavefronts (253 x 231 x 246 torus, MP5, after 70 substeps: 11.6 ms a
 // substep with the queue, 8.73 so; 64^3 WENO-Z 0.219 -> 0.192 ms; 22 x 17 x 13
-// con2prim 50 -> 26 us; 192^3, no failed zones: the same).
+// con2prim 50 -> 26 us; 192^3, no failed zones: the same), and where they are
+// scattered too (con2prim of 128^3, a twentieth of the primaries failed at
+// random: 0.80 -> 0.61 ms).
 template <bool FROM_A, class E>
 __global__ __launch_bounds__(256) void k_c2p_one(KPatch P, Box B, E eos, C2PArgs a,
                                                  unsigned long long *hist) {
@@ -156,10 +158,12 @@ __global__ __launch_bounds__(256) void k_c2p_patches(const KPatch *__restrict__ 
 // Independent zones (layout of asx_c2p_batch in include/asterx.h) in two
 // passes without scratch memory: every zone through the primary solver, which
 // alone sets the register budget (124 VGPRs for Noble and 114 for Palenzuela,
-// 4 waves per SIMD; 241 and 2 for the full chain); a zone it fails gets the flag kZoneFailed,
-// which the second pass looks for.  Bound by the latency of the Newton
+// 4 waves per SIMD; 241 and 2 for the full chain); a zone it fails gets the
+// flag kZoneFailed, which the second pass looks for, and in iters the steps
+// of a Newton chain that did not converge, which is not repeated then (-1
+// for any other failure).  Bound by the latency of the Newton
 // steps' dependent square roots and reciprocals: 4 000 037 zones from the
-// previous step's primitives 0.770 -> 0.470 ms (0.13 of them the second pass).
+// previous step's primitives 0.770 -> 0.427 ms (0.10 of them the second pass).
 constexpr double kZoneFailed = -1.0;
 template <int PRIME>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
@@ -175,13 +179,15 @@ void k_c2p_zones(int64_t nz, const double *cons, const double *g, const double *
     iters[z] = o.iters;
   } else {
     flag[z] = kZoneFailed;
+    iters[z] = PRIME == ASX_C2P_NOBLE && o.failed == ST_ROOT_FAIL_CONV ? o.iters : -1;
   }
 }
-// The failed zones among each wavefront's `per` <= kRestZones, gathered in LDS, through
-// the full chain: a chain of thirty failed Newton steps and the backup's
+// The failed zones among each wavefront's `per` <= kRestZones, gathered in
+// LDS, through the rest of the chain: the latency of the backup's
 // iterations, so what counts is that the few zones spread over all SIMDs
-// (4 000 037 zones: 0.19 ms with workgroups of 256 for 4096 zones, 0.13 with
-// a wavefront each).
+// (4 000 037 zones, the failed Newton steps repeated as well: 0.19 ms with
+// workgroups of 256 for 4096 zones, 0.13 with a wavefront each; 0.10 without
+// the Newton steps).
 constexpr int kRestZones = 4096;
 __global__ __launch_bounds__(64)
 void k_c2p_zones_rest(int64_t nz, int per, const double *cons, const double *g,
@@ -202,7 +208,7 @@ void k_c2p_zones_rest(int64_t nz, int per, const double *cons, const double *g,
     C2PIn in;
     batch_zone_in(z, nz, cons, g, seed, a, in);
     C2POut o;
-    con2prim_cell(eos, a, in, o);
+    con2prim_cell(eos, a, in, o, -1.0, -1.0, iters[z]);
     batch_zone_out(z, nz, o, prim, flag);
     iters[z] = o.iters;
   }

@@ -340,10 +340,12 @@ ASX_DEV void vel_from_Z(double Z, double W, double Bsq, double BiSi, const Cons 
 // replace the seed-derived initial guess (used by the learned guess).
 // SEEDLESS: the guess is given (zguess >= 0) and the seed is not read at
 // all (the saved primitives need not be loaded); same iterates otherwise.
+// spent: see con2prim_zone.
 template <bool SEEDLESS = false>
 ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a,
                          Prim &pv, Prim &seed, Cons &cv, const Sym3 &glo,
-                         Report &rep, double zguess = -1.0, double vguess = -1.0) {
+                         Report &rep, double zguess = -1.0, double vguess = -1.0,
+                         int spent = -1) {
   rep.iters = 0;
   rep.adjust_cons = false;
   rep.set_atmo = false;
@@ -403,6 +405,12 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
         (seed.rho + eps_last * seed.rho + seed.press) * seed.w_lor * seed.w_lor;
     x0 = fabs(Z_seed);
     x1 = vsq_seed;
+  }
+  if (spent >= 0) { // known not to converge: as the loop leaves
+    rep.iters = spent;
+    rep.status = ST_ROOT_FAIL_CONV; rep.adjust_cons = true;
+    cv.scale(sqrt_detg);
+    return;
   }
   if (zguess >= 0.0) {
     x0 = zguess;
@@ -855,15 +863,20 @@ struct C2POut {
   Cons cv;
   double flag, mask_cc;
   int iters;
+  int failed; // status of a primary-only solve that failed
 };
 
 // AsterX/src/con2prim.cxx:81-416.
 // PRIME < 0: the full chain, primary and backup solver chosen at run time
 // from a.prime / a.second (the reference's behaviour); returns true.
 // PRIME = ASX_C2P_NOBLE or ASX_C2P_PALENZUELA: only the primary solver,
-// compiled for that method (a.prime must equal it); returns false, with
-// `out` not set, when it fails: the zone then needs the full chain, which
-// repeats the same primary solve before the backup.
+// compiled for that method (a.prime must equal it); returns false when it
+// fails, with out.iters and out.failed set and nothing else: the zone then
+// needs the full chain, which repeats the same primary solve before the
+// backup.  On a table without a backup (and without a guess that the full chain
+// would do without) the chain ends here: true, as by the full chain.
+// spent >= 0 (full chain): the primary is known to have failed to converge in
+// so many iterations, and its loop is not repeated.
 // zguess, vguess (optional, > 0) guide the primary solver: Noble starts
 // from Z = zguess, v^2 = vguess; Palenzuela brackets x = h W within the
 // relative half-width vguess of zguess when the residual changes sign
@@ -874,7 +887,8 @@ struct C2POut {
 // otherwise.
 template <int PRIME, class E, bool SEEDLESS = false>
 ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
-                           C2POut &out, double zguess = -1.0, double vguess = -1.0) {
+                           C2POut &out, double zguess = -1.0, double vguess = -1.0,
+                           int spent = -1) {
   static_assert(!SEEDLESS || PRIME == ASX_C2P_NOBLE, "seedless: the Noble primary only");
   const Atmo atmo = make_atmo(eos, a, in.r);
   const Sym3 &glo = in.glo;
@@ -941,7 +955,7 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
     const int prime = PRIME < 0 ? a.prime : PRIME;
     if constexpr (std::is_same<E, IdealGas>::value) {
       if (prime == ASX_C2P_NOBLE)
-        noble_solve<SEEDLESS>(eos, atmo, a, pv, seed, cv, glo, rep1, zguess, vguess);
+        noble_solve<SEEDLESS>(eos, atmo, a, pv, seed, cv, glo, rep1, zguess, vguess, spent);
       else if (prime == ASX_C2P_ENTROPY) entropy_solve(eos, atmo, a, pv, cv, glo, rep1);
       else palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, in.temperature, zguess, vguess, PRIME >= 0);
     } else {
@@ -949,13 +963,14 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
       palenzuela_solve(eos, atmo, a, pv, cv, glo, rep1, in.temperature, zguess, vguess, PRIME >= 0);
     }
     out.iters = rep1.iters;
-    // On a table without a backup the chain ends here (no guess that a second
-    // solve would do without): the zone need not repeat a primary of up to
-    // max_iter temperature solves to find that out.
+    // (on the ideal gas the atmosphere's and the black hole's code beside the
+    // solver would cost a wave per SIMD)
     constexpr bool ends = !std::is_same<E, IdealGas>::value;
     if (PRIME >= 0 && rep1.failed() &&
-        !(ends && zguess < 0.0 && a.second != ASX_C2P_PALENZUELA))
+        !(ends && zguess < 0.0 && a.second != ASX_C2P_PALENZUELA)) {
+      out.failed = rep1.status;
       return false;
+    }
     if (rep1.failed()) code = ASX_C2P_FLAG_SECOND;
     if (PRIME < 0 && rep1.failed()) {
       if constexpr (std::is_same<E, IdealGas>::value) {
@@ -996,8 +1011,8 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
 }
 template <class E>
 ASX_DEV void con2prim_cell(const E &eos, const C2PArgs &a, const C2PIn &in, C2POut &out,
-                           double zguess = -1.0, double vguess = -1.0) {
-  (void)con2prim_zone<-1>(eos, a, in, out, zguess, vguess);
+                           double zguess = -1.0, double vguess = -1.0, int spent = -1) {
+  (void)con2prim_zone<-1>(eos, a, in, out, zguess, vguess, spent);
 }
 
 // Append `value` of every work-item with `fail` set to the queue: a

@@ -323,12 +323,17 @@ hipError_t launch_con2prim_one(const KPatch &P, const TabEOS &eos, const C2PArgs
                                bool from_A, unsigned long long *hist, hipStream_t s);
 // Independent zones, whose failures are scattered, take one pass while all
 // wavefronts are resident at the full chain's two per SIMD (2 x 4 x 256 of
-// 64): its registers then cost nothing, and the second pass is saved.
+// 64): its registers then cost nothing, and the second pass is saved.  One
+// pass / two, Noble with a Palenzuela backup: at this line 63 / 67 us where the
+// primary fails 5 zones in 10^4, 22.8 / 23.3 where it fails none; 200 000 zones
+// 75 / 86 and 38 / 31; 10^6 zones 212 / 179 and 130 / 92.
 constexpr int64_t kOnePassZones = 128 * 1024;
 // A patch on a table takes the two passes below beyond this many zones: the
-// table's full chain is the slower body (128^3 substep 2.33 ms in one pass,
-// 2.15 in two; 90^3 0.85 / 0.79, 44^3 0.142 / 0.134, 64^3 0.256 / 0.266), and
-// below a wavefront per SIMD the launches saved weigh more.
+// table's full chain is the slower body, and below a wavefront per SIMD the
+// launches saved weigh more.  Substep in one pass / two, without a backup: 32^3
+// 94 / 102 us, 40^3 118 / 126, 44^3 143 / 135, 64^3 329 / 315, 90^3 859 / 790,
+// 128^3 2350 / 2123; after a hundred substeps, whose zones iterate less, 64^3
+// 259 / 266 and 90^3 685 / 686.
 constexpr int64_t kOnePassTableZones = 64 * 1024;
 // con2prim of the patch interior in two passes: every zone through the
 // primary solver, the zones it failed queued (queue: one int per interior

@@ -40,7 +40,9 @@ def _solve(par, cons, g, seed):
     return prim.cpu().numpy(), flag.cpu().numpy(), it.cpu().numpy()
 
 
-@pytest.mark.parametrize("prime,second", [("Noble", "Palenzuela"), ("Palenzuela", "Noble")])
+@pytest.mark.parametrize("prime,second", [("Noble", "Palenzuela"), ("Palenzuela", "Noble"),
+                                          ("Noble", "Noble"), ("Noble", "None"),
+                                          ("Noble", "None+fix"), ("Entropy", "None")])
 @pytest.mark.parametrize("nz", [ONE_PASS, ONE_PASS + 1, ONE_PASS + 4160])
 def test_zones(prime, second, nz):
     from asterx_amd.zones import make_batch
@@ -53,7 +55,8 @@ def test_zones(prime, second, nz):
     cons[0, 1::1999] = 1e-14
     cons[4, 2::1501] = np.inf
     par = abi.params(gl_gamma=5.0 / 3.0, eps_max=1e8, rho_max=1e8, rho_abs_min=1e-12,
-                     vw_lim=1e3, B_lim=1e3, c2p_prime=prime, c2p_second=second)
+                     vw_lim=1e3, B_lim=1e3, c2p_prime=prime, c2p_second=second.split("+")[0],
+                     use_entropy_fix=int("+fix" in second))
     one = _solve(par, cons, g, seed)
     reps = -(-nz // n0)
     two = _solve(par, *(np.tile(a, (1, reps))[:, :nz] for a in (cons, g, seed)))
