@@ -27,9 +27,10 @@ ASX_DEV void hist_flush(HistLDS &h, unsigned long long *g) {
 }
 
 // Pass 1: every zone through the primary solver (Palenzuela, the only one a
-// table takes; compiled alone, so the backup costs no registers here).  Zones
-// whose primary solve fails store nothing; a wavefront ballot packs their
-// indices into `queue` with one atomic per wavefront.
+// table takes; compiled alone, so the backup costs no registers here).  Where
+// there is a backup, zones whose primary solve fails store nothing; a wavefront
+// ballot packs their indices into `queue` with one atomic per wavefront.
+// Without one they end here, and the queue stays empty.
 template <bool FROM_A, class E>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(c2p_waves<E>())))
 void k_c2p_main(KPatch P, Box B, E eos, C2PArgs a, unsigned long long *hist, int *queue,

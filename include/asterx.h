@@ -316,11 +316,12 @@ enum {
   ASX_KC_AUX = 4,    /* vertex auxiliaries of the A/Psi gauge (batch plans;
                         on one patch they ride on the face launches) */
   ASX_KC_UPDATE = 5, /* fused RHS + RK combination */
-  ASX_KC_C2P = 6,    /* con2prim: every zone, primary solver (patch or batch) */
+  ASX_KC_C2P = 6,    /* con2prim: the full chain of every zone, or the primary
+                        solver where the zones it fails follow (C2P_REST) */
   ASX_KC_BC = 7,     /* boundary fills */
   ASX_KC_RHS = 8,    /* unfused source terms / RHS */
   ASX_KC_OTHER = 9,
-  ASX_KC_C2P_REST = 10, /* con2prim: zones the primary solver failed */
+  ASX_KC_C2P_REST = 10, /* con2prim of a large table patch: zones the primary failed */
   ASX_KC_MLP = 11,      /* learned con2prim guess: inference and training */
   ASX_KC_GRAPH = 12,    /* replays of a batch plan's captured step */
   ASX_KC_TMUNU = 13,    /* stress-energy tensor at the vertices */
@@ -662,7 +663,10 @@ asx_status asx_mlp_train_step(int64_t nz, const double *cons, const double *g,
  * the matrix cores inside the primary-solver kernel, so the guesses never
  * reach memory; variant 1 runs the forward pass as a kernel of its own and
  * keeps the guesses in library scratch.  The queue of unconverged zones
- * lives in library scratch per device and stream, grown on demand. */
+ * lives in library scratch per device and stream, grown on demand.
+ * When to prefer it: on 2^24 zones it runs at 0.87 times asx_c2p_batch's rate
+ * from cold seeds and 1.01 times from the previous step's (variant 1: 0.75 and
+ * 0.89), so only where the plain seed makes many primaries fail. */
 asx_status asx_c2p_batch_mlp(int64_t nz, const double *cons, const double *g,
                              const double *seed, const float *blob, int32_t kguess,
                              double *prim, double *flag, int32_t *iters, int32_t *fallback,
@@ -694,8 +698,9 @@ asx_status asx_prim2con_batch_ye(int64_t nz, const double *prim, const double *g
  * prim[9][nz] = the asx_c2p_batch rows, then Ye.  With a table: Palenzuela
  * (c2p_prime), use_temperature = yes and use_press_atmo = no, as the
  * reference's table requires (eps_from_valid_rho_press_ye is refused there).
- * Two passes as asx_con2prim (primary solver, then the queue of the zones
- * it failed through the full chain); nz < 2^31. */
+ * Two passes (primary solver, then the queue of the zones it failed through
+ * the full chain; the queue lives in library scratch per device and stream,
+ * grown on demand); nz < 2^31. */
 asx_status asx_c2p_batch_ye(int64_t nz, const double *cons, const double *g,
                             const double *seed, double *prim, double *flag, int32_t *iters,
                             const asx_params *par, void *stream);
@@ -739,7 +744,9 @@ asx_status asx_mlp_ye_train_step(int64_t nz, const double *cons, const double *g
  * (inside the widest bracket the reference may take) when the residual
  * changes sign there, and takes the reference's bracket otherwise; the
  * root, hence the result, is the same to the solver tolerance.
- * 0 < bracket < 1.  The guesses and the queue live in library scratch per
+ * 0 < bracket < 1.  It takes a quarter fewer Brent iterations than
+ * asx_c2p_batch_ye and runs at 0.98 times its rate (2^22 zones, seeds from the
+ * previous step).  The guesses and the queue live in library scratch per
  * device and stream.  An ideal gas returns ASX_ERR_UNSUPPORTED (use
  * asx_c2p_batch_mlp). */
 asx_status asx_c2p_batch_ye_mlp(int64_t nz, const double *cons, const double *g,
