@@ -2435,6 +2435,21 @@ asx_status plan_persist_prepare(asx_batch *b) {
     out = BatchList{L->box, L->map, L->nmap};
     return true;
   };
+  // first global zone of each patch, and the queue of the zones the primary fails
+  if (!b->queue) {
+    std::vector<int> zb(b->np + 1, 0);
+    for (int p = 0; p < b->np; ++p) {
+      const int32_t *n = b->pt[p].n;
+      zb[p + 1] = zb[p] + n[0] * n[1] * n[2];
+    }
+    void *q = nullptr, *qc = nullptr;
+    if ((st = plan_upload(b, zb, &b->zbase))) return st;
+    if (plan_alloc(b, sizeof(unsigned), &qc) != hipSuccess ||
+        plan_alloc(b, (size_t)b->nzones * sizeof(int), &q) != hipSuccess)
+      return ASX_ERR_DEVICE;
+    b->qcount = (unsigned *)qc;
+    b->queue = (int *)q;
+  }
   PersistArgs a;
   std::memset(&a, 0, sizeof(a));
   for (int d = 0; d < 3; ++d)
@@ -2597,21 +2612,11 @@ asx_status asx_batch_create(int32_t npatch, const asx_patch *patches, const asx_
       sp[k].push_back(P);
     }
   }
-  std::vector<int> zb(npatch + 1, 0);
-  for (int p = 0; p < npatch; ++p)
-    zb[p + 1] = zb[p] + patches[p].n[0] * patches[p].n[1] * patches[p].n[2];
   for (int k = 0; k < 3 && !st; ++k)
     if (!(st = plan_upload(b, stab[k], &b->stab[k])) &&
         !(st = plan_upload(b, utab[k], &b->utab[k])))
       st = plan_upload(b, sp[k], &b->st[k]);
-  if (!st) st = plan_upload(b, zb, &b->zbase);
   if (st) return fail(st);
-  void *q = nullptr, *qc = nullptr;
-  if (plan_alloc(b, (size_t)zones * sizeof(int), &q) != hipSuccess ||
-      plan_alloc(b, sizeof(unsigned), &qc) != hipSuccess)
-    return fail(ASX_ERR_DEVICE);
-  b->queue = (int *)q;
-  b->qcount = (unsigned *)qc;
   if ((st = plan_prepare(b))) return fail(st);
   *plan = b;
   return ASX_OK;

@@ -771,7 +771,8 @@ asx_status asx_c2p_batch_ye_mlp(int64_t nz, const double *cons, const double *g,
  * Requirements per patch are those of asx_substep and asx_con2prim_group;
  * ghost zones are filled with `bc_kind` on every face (there is no
  * inter-patch exchange).  The plan owns the face/aux scratch of all
- * patches and the con2prim queue; it holds the descriptors, not the data. */
+ * patches (and, from the first persistent step on, that form's launch lists
+ * and con2prim queue); it holds the descriptors, not the data. */
 typedef struct asx_batch_s asx_batch;
 asx_status asx_batch_create(int32_t npatch, const asx_patch *patches, const asx_state *bufs,
                             const asx_params *par, double dt, int32_t bc_kind,

@@ -161,6 +161,25 @@ def test_persistent_stage_matches_plain_launches(recon):
             abi.check("asx_set_variant", L.asx_set_variant(kc, v))
 
 
+def test_failed_zone_queue_is_the_persistent_stage_s():
+    """Plain launches and graphs run the full chain in each zone's lane: the
+    queue (4 bytes a zone) is allocated with the first persistent step."""
+    torch = _torch()
+    pa, par, dt = _cuts(seed=5)
+    plan = batch.Plan(_L(), pa, par, dt)
+    zones = sum(p.n[0] * p.n[1] * p.n[2] for p in pa)
+    plan.step(1, graph=True)
+    before = plan.info()[1]
+    plan.step(1, persistent=True)
+    torch.cuda.synchronize()
+    assert plan.info()[0] == zones and plan.info()[1] >= before + 4 * zones
+    more = plan.info()[1]
+    plan.step(1, persistent=True)
+    torch.cuda.synchronize()
+    assert plan.info()[1] == more
+    plan.close()
+
+
 def test_persistent_stage_refuses_unsupported():
     """Methods the persistent stage is not built for are refused, not run."""
     _torch()
