@@ -135,11 +135,11 @@ def build(nrho=NRHO, ntemp=NTEMP, nye=NYE):
     return code_units(*make_cgs(nrho, ntemp, nye))
 
 
-def eps_grows_with_T(data):
+def eps_grows_with_T(data, axes):
     """Whether log(eps + shift) grows by more than 1e-12 (well above the
     rounding of an interpolation) from every T node to the next: then one T
     has a given eps, and a solve may start its search anywhere."""
-    le = data[..., 1]
+    le = np.reshape(data, [len(a) for a in axes[::-1]] + [4])[..., 1]
     return bool(np.all(le[:, 1:] - le[:, :-1] > 1e-12))
 
 
@@ -193,7 +193,7 @@ class Table:
             d.x_lo[k] = float(a[0])
             d.x_step[k] = float(a[1] - a[0])
             d.x_hi[k] = float(a[-1])
-        d.eps_grows_with_T = eps_grows_with_T(tab["data"])
+        d.eps_grows_with_T = eps_grows_with_T(tab["data"], tab["axes"])
         self.desc = d
 
     def attach(self, par):

@@ -117,5 +117,7 @@ def test_growth_with_temperature(tmp_path, node):
     assert L.asx_eos_read_stellarcollapse(path.encode(), C.byref(t)) == 0
     assert t.eps_grows_with_T == (node is None)
     L.asx_eos_host_table_free(C.byref(t))
-    host = tabeos.Table(tabeos.read_stellarcollapse(path), device=None)
-    assert host.desc.eps_grows_with_T == (node is None)
+    tab = tabeos.read_stellarcollapse(path)
+    for data in (tab["data"], tab["data"].ravel()):
+        host = tabeos.Table(dict(tab, data=data), device=None)
+        assert host.desc.eps_grows_with_T == (node is None)
