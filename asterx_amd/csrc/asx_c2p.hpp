@@ -282,10 +282,10 @@ ASX_DEV void bh_interior(const E &eos, const Atmo &atmo, const C2PArgs &a,
 }
 
 // c2p::cons_floors_and_ceilings (Con2PrimFactory/src/c2p.hxx:330-369)
-ASX_DEV void cons_floors(Cons &cv, const Sym3 &glo) {
+template <bool SPLIT> ASX_DEV void cons_floors(Cons &cv, const Sym3 &glo) {
   const double detg = det3(glo);
   const double sqrt_detg = sqrt(detg);
-  const Sym3 gup = inv3(glo, detg);
+  const Sym3 gup = inv3<SPLIT>(glo, detg);
   double B_low[3];
   lower(glo, cv.dB, B_low);
   const double tau_lim = 0.5 * dot3(B_low, cv.dB) / sqrt_detg;
@@ -359,7 +359,7 @@ ASX_DEV void noble_solve(const IdealGas &eos, const Atmo &atmo, const C2PArgs &a
     prim_nan(pv); cv.set_nan();
     return;
   }
-  const Sym3 gup = inv3(glo, detg);
+  const Sym3 gup = inv3<!SEEDLESS>(glo, detg);
   cv.divide(sqrt_detg);
   seed.B[0] = cv.dB[0]; seed.B[1] = cv.dB[1]; seed.B[2] = cv.dB[2];
   double mom_up[3], B_low[3];
@@ -948,7 +948,7 @@ ASX_DEV bool con2prim_zone(const E &eos, const C2PArgs &a, const C2PIn &in,
     call_c2p = false;
   }
   Report rep1{ST_NOT_SET, false, false, 0}, rep2{ST_NOT_SET, false, false, 0};
-  cons_floors(cv, glo);
+  cons_floors<!SEEDLESS>(cv, glo);
   out.iters = 0;
   if (call_c2p) {
     code = ASX_C2P_FLAG_PRIME;

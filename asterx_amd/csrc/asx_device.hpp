@@ -116,17 +116,25 @@ ASX_DEV double det3(const Sym3 &g) {
   return 2 * g.xy * g.xz * g.yz + g.xx * g.yy * g.zz - g.yy * pow2(g.xz) -
          g.xx * pow2(g.yz) - g.zz * pow2(g.xy);
 }
-// The branch ends the live ranges before it (con2prim of independent zones
-// 152 -> 124 VGPRs); quotients put right afterwards where they do not hold cost
-// con2prim of a patch its second wave per SIMD (192^3 substep 4.41 -> 5.03 ms).
-ASX_DEV Sym3 inv3(const Sym3 &g, double det) {
+// SPLIT: a branch for each kind of divisor, which ends the live ranges before
+// it (con2prim of independent zones 152 -> 124 VGPRs).  Else the quotients in
+// line with what surrounds them, put right afterwards where they do not hold:
+// for the guided solve, whose registers suffice (2^24 zones 1.36 -> 1.33 ms); con2prim of
+// a patch loses its second wave per SIMD (192^3 substep 4.41 -> 5.03 ms).
+template <bool SPLIT = true> ASX_DEV Sym3 inv3(const Sym3 &g, double det) {
   auto over = [&](const auto &d) {
     return Sym3{(g.yy * g.zz - pow2(g.yz)) / d, (g.xz * g.yz - g.xy * g.zz) / d,
                 (g.xy * g.yz - g.xz * g.yy) / d, (g.xx * g.zz - pow2(g.xz)) / d,
                 (g.xy * g.xz - g.xx * g.yz) / d, (g.xx * g.yy - pow2(g.xy)) / d};
   };
   const Divisor d(det);
-  return d.holds() ? over(d) : over(det);
+  if constexpr (SPLIT) {
+    return d.holds() ? over(d) : over(det);
+  } else {
+    Sym3 u = over(d);
+    if (!d.holds()) u = over(det);
+    return u;
+  }
 }
 ASX_DEV void lower(const Sym3 &g, const double v[3], double o[3]) {
   o[0] = 0.0 + g.xx * v[0] + g.xy * v[1] + g.xz * v[2];
